@@ -69,6 +69,8 @@ const char *rvkv_last_error(void);
  * (the reference's own cell type): an f32 pool supports append (f32 rows
  * copied, f16 rows widened exactly), gather into F32 only, copy_blocks,
  * read_blocks, block_checksums, attn_prep, paged decode and paged prefill.
+ * The same allocation ends in 32 MiB of scratch for rvkv_paged_prefill (left
+ * out if there is no room for it).
  * The pool binds to the current HIP device and to `stream`. */
 int rvkv_pool_create(uint32_t n_layers, uint32_t num_blocks,
                      uint32_t block_size, uint32_t n_kv_heads,
@@ -306,7 +308,11 @@ int rvkv_attn_prep(rvkv_pool *pool, uint32_t layer, const float *q_in,
  * head_dim in {32, 64, 128, 256} and block_size a power of two >= 8 it is
  * computed on the matrix cores in f16 with f32 accumulation; any other
  * head_dim <= 1024, block size or an f32 pool runs a generic kernel in f32
- * arithmetic. Allocates nothing. */
+ * arithmetic. Allocates nothing. Calls whose query rows alone leave the GPU
+ * idle are cut along the keys and merged by a second launch; the partial
+ * results go to the pool's scratch, half of which the first two streams that
+ * such calls run on get each. On further streams, and under graph capture,
+ * the keys are not cut (the same result to within rounding). */
 int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
                        const uint32_t *block_tables,
                        const uint32_t *pos_offset,

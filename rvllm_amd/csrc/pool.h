@@ -24,6 +24,14 @@ struct rvkv_pool {
   size_t tensor_elems;   // num_blocks * n_kv * block_size * head_dim
   size_t block_elems;    // n_kv * block_size * head_dim
   size_t tensor16, block16;
+  // Scratch for the partial results of prefills that are cut along their
+  // keys: kSplitStreams regions of kSplitBytes behind the cache tensors, in
+  // the same allocation (NULL if there was no room for them). A region
+  // belongs to the first stream that used it, for the pool's life, so two
+  // streams never share one and calls need no ordering between streams.
+  unsigned char *split_base;
+  hipStream_t split_stream[2];
+  uint32_t n_split;
 
   uint16_t *tensor(uint32_t layer, uint32_t which) const {
     return base + ((size_t)layer * 2 + which) * tensor16;
@@ -32,6 +40,12 @@ struct rvkv_pool {
 };
 
 namespace rvkv_detail {
+constexpr size_t kSplitBytes = (size_t)16 << 20;
+constexpr uint32_t kSplitStreams = 2;
+// The scratch region of the pool's current stream; NULL when every region
+// belongs to another stream, or while the stream is captured (a graph may be
+// replayed beside any later call): the caller then does without.
+void *split_scratch(rvkv_pool *pool);
 // Records "<op>: <reason>" as the last error and returns code.
 int fail(int code, const char *op, const char *reason);
 // Records "<op>: <HIP error string>" and returns RVKV_EHIP.

@@ -39,6 +39,7 @@
 // f32; sums are f32.
 #include "pool.h"
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdlib>
@@ -46,6 +47,7 @@
 
 using rvkv_detail::fail;
 using rvkv_detail::hip_fail;
+using rvkv_detail::kSplitBytes;
 
 namespace {
 
@@ -152,6 +154,11 @@ struct PrefillArgs {
   // dec_ctx_cap, as the VALU decode's uniform mode does.
   uint32_t dec_parts, dec_part_tokens, dec_ctx_cap;
   float *ws_acc, *ws_ml;
+  // Prefill with a tile's keys cut into pieces of split_keys (a multiple of
+  // the key tile; 0: not cut), split_n the most pieces a tile can have:
+  // grid = pieces x query tiles. Piece i of a tile with more than one writes
+  // its partial to ws_acc / ws_ml [i][q row]; prefill_reduce_kernel merges.
+  uint32_t split_keys, split_n;
   // Fused append (decode mode): this step's K/V row of every sequence
   // ([batch, n_kv, hd], f32 or f16) goes to slot (new_blk[b], new_off[b])
   // and is the key at position ctx - 1; the work item holding that key
@@ -266,6 +273,24 @@ __device__ __forceinline__ uint32_t lo_bound(uint32_t p, int32_t window) {
                                                   : 0u;
 }
 
+// The keys [begin, end) that the rows of query tile `tile` of sequence b see
+// in a prefill, begin on a key-tile boundary; shared by the prefill kernel
+// and its reduction, which must agree on a tile's pieces.
+struct KeyRange {
+  uint32_t begin, end;
+  __device__ uint32_t pieces(uint32_t split_keys) const {
+    return end > begin ? (end - begin + split_keys - 1) / split_keys : 0u;
+  }
+};
+template <int BM, int BN>
+__device__ __forceinline__ KeyRange tile_keys_of(const PrefillArgs &a,
+                                                 uint32_t off, uint32_t ctx,
+                                                 uint32_t tile, uint32_t rows) {
+  const uint32_t r0 = tile * BM, r1 = min(r0 + BM, rows) - 1u;
+  return {lo_bound(off + r0 / a.group, a.window) & ~(uint32_t)(BN - 1),
+          min(ctx, off + r1 / a.group + 1u)};
+}
+
 // WAVES wave64s per workgroup (4 or 8, 32 query rows each); the K/V tile
 // loads and LDS stores are shared among them, so more waves halve each
 // wave's share of that work. Registers are bounded for 8 resident waves per
@@ -275,7 +300,9 @@ __device__ __forceinline__ uint32_t lo_bound(uint32_t p, int32_t window) {
 // matrix work. (With all of O and Q in one wave, head_dim 256 ran one wave
 // per SIMD, its S product serialised on LDS reads: 18 % slower. 128-key
 // tiles at head_dim 64 were measured 7-9 % slower than 64.)
-template <int HD, int WAVES, int KSPLIT = 1>
+// One-wave workgroups are the decode's, the others the prefill's, so each
+// kernel holds only its own work split; CUT: query tiles' keys in pieces.
+template <int HD, int WAVES, int KSPLIT = 1, bool CUT = false>
 __global__ void __launch_bounds__(
     64 * WAVES * KSPLIT,
     // (a one-wave workgroup may share a SIMD with others: 2 bounds the
@@ -283,6 +310,7 @@ __global__ void __launch_bounds__(
     WAVES == 1 ? 2 : (HD <= 64 ? 12 : 8) / WAVES)
     prefill_kernel(PrefillArgs a) {
   constexpr int NTH = 64 * WAVES;  // threads per workgroup
+  constexpr bool DEC = WAVES == 1;
   constexpr bool SPLIT = split_dims(HD);
   static_assert(!SPLIT || (WAVES % 2 == 0 && WAVES > 1), "wave pairs");
   constexpr int kBM = block_rows<HD, WAVES>();
@@ -333,11 +361,12 @@ __global__ void __launch_bounds__(
   // K/V, which then stays in that XCD's L2. Within a head, long (late)
   // rows go first.
   uint32_t tile, kvh, b, item_lo = 0, item_hi = 0xFFFFFFFFu, slot = kNoSlot;
+  uint32_t piece = 0;  // of a prefill tile's keys (a.split_keys)
   // Group item: member list (n, sequences, slots); its first member's
   // table serves every member over the item's range.
   const uint32_t *gl = nullptr;
   uint32_t n_mem = 0;
-  if (a.items) {  // decode items: grid (items, n_kv), plan order kept
+  if (DEC && a.items) {  // decode items: grid (items, n_kv), plan order kept
     typedef const __attribute__((address_space(4))) uint32_t cu32;
     cu32 *itp = (cu32 *)(uintptr_t)(a.items + blockIdx.x);  // scalar loads
     const uint4 it = make_uint4(itp[0], itp[1], itp[2], itp[3]);
@@ -352,7 +381,7 @@ __global__ void __launch_bounds__(
       n_mem = gl[0];
       b = gl[1];
     }
-  } else if (a.dec_parts) {  // uniform decode partitions
+  } else if (DEC && a.dec_parts) {  // uniform decode partitions
     b = blockIdx.x / a.dec_parts;
     const uint32_t part = blockIdx.x - b * a.dec_parts;
     item_lo = part * a.dec_part_tokens;
@@ -371,15 +400,23 @@ __global__ void __launch_bounds__(
     }
     tile = 0;
   } else {
-    const uint32_t n_wg = a.n_tiles * a.n_kv * a.batch;
+    const uint32_t n_wg = gridDim.x;
     const uint32_t w = blockIdx.x, xcd = w % 8, idx = w / 8;
     const uint32_t per = n_wg / 8, rem = n_wg % 8;
-    const uint32_t logical =
+    uint32_t logical =
         xcd < rem ? xcd * (per + 1) + idx
                   : rem * (per + 1) + (xcd - rem) * per + idx;
+    // (Pieces: a causal prompt's late pieces hold fewer tiles, so a head
+    // spread over several XCDs goes round robin.)
+    if (CUT && (a.n_kv * a.batch) % 8 != 0) logical = w;
     tile = a.n_tiles - 1 - logical % a.n_tiles;
-    kvh = (logical / a.n_tiles) % a.n_kv;
-    b = logical / a.n_tiles / a.n_kv;
+    uint32_t rest = logical / a.n_tiles;
+    if (CUT) {  // the tiles of one piece re-read the same K/V
+      piece = rest % a.split_n;
+      rest /= a.split_n;
+    }
+    kvh = rest % a.n_kv;
+    b = rest / a.n_kv;
   }
   const int tid = KSPLIT > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -393,22 +430,31 @@ __global__ void __launch_bounds__(
   // sequence wraps to 2^32 - 1 and sees no key).
   // (b is uniform: the per-sequence words come by scalar loads)
   typedef const __attribute__((address_space(4))) uint32_t cu32s;
-  const bool decode = a.items || a.dec_parts;
-  const uint32_t rn = a.dec_parts
+  const uint32_t rn = DEC && a.dec_parts
                           ? min(*(cu32s *)(uintptr_t)(a.read_num + b),
                                 a.dec_ctx_cap)
                           : *(cu32s *)(uintptr_t)(a.read_num + b);
   const uint32_t off =
-      decode ? rn - 1u : *(cu32s *)(uintptr_t)(a.pos_offset + b);
+      DEC ? rn - 1u : *(cu32s *)(uintptr_t)(a.pos_offset + b);
   const uint32_t cap = a.max_blocks << a.bs_log2;
   const uint32_t ctx = min(rn, cap);
-  if (a.dec_parts) {
+  if (DEC && a.dec_parts) {
     // One partition covers the sequence: its output is written directly
     // (the reduction skips it). A partition past the sequence's end has
     // nothing to do (the reduction never reads it); an empty sequence gets
     // its zero row from partition 0.
     if (ctx <= a.dec_part_tokens) slot = kNoSlot;
     if (item_lo >= ctx && item_lo > 0) return;
+  }
+  if constexpr (CUT) {
+    const KeyRange kr = tile_keys_of<kBM, BN>(a, off, ctx, tile, a.rows);
+    const uint32_t np = kr.pieces(a.split_keys);
+    if (piece >= np && piece > 0) return;  // (the reduction skips it)
+    if (np > 1) {
+      slot = piece;
+      item_lo = kr.begin + piece * a.split_keys;
+      item_hi = item_lo + a.split_keys;
+    }
   }
   if constexpr (KSPLIT > 1) {
     // This wave's share of the item's keys, in whole tiles (item_lo is a
@@ -463,7 +509,7 @@ __global__ void __launch_bounds__(
   const size_t qrow = ((size_t)bq * a.q_len + qi) * a.n_heads + head;
   // The appended key (fused decode step) when this item holds it.
   const uint32_t newtok =
-      (a.new_k && ctx >= 1u && ctx - 1u >= item_lo && ctx - 1u < item_hi)
+      (DEC && a.new_k && ctx >= 1u && ctx - 1u >= item_lo && ctx - 1u < item_hi)
           ? ctx - 1u
           : 0xFFFFFFFFu;
 
@@ -1094,9 +1140,12 @@ __global__ void __launch_bounds__(
     }
   }
   const float lt = sum_halves(l);
-  if (gl || slot != kNoSlot) {  // split decode sequences: partials
+  if (gl || slot != kNoSlot) {  // split sequences or tiles: partials
     if (row_ok) {
-      const size_t idx = (size_t)my_slot * a.n_heads + head;
+      // (a prefill piece: [piece][q row])
+      const size_t idx =
+          CUT ? (size_t)slot * a.batch * a.q_len * a.n_heads + qrow
+              : (size_t)my_slot * a.n_heads + head;
       float *op = a.ws_acc + idx * HD;
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
@@ -1127,8 +1176,72 @@ __global__ void __launch_bounds__(
   }
 }
 
+// Merges the pieces of the query tiles that prefill_kernel cut: HD / 4 lanes
+// of a q row (token, head), four elements each; weights 2^(m_i - M). Rows of
+// uncut tiles are left alone (the prefill kernel wrote them). Bound by the
+// launch and the round trips to the partials: eight pieces' (m, l) and
+// partials are loaded at a time.
 template <int HD, int WAVES>
-void launch_prefill(const PrefillArgs &a, dim3 grid, hipStream_t st) {
+__global__ void __launch_bounds__(256)
+    prefill_reduce_kernel(PrefillArgs a, uint32_t n_rows) {
+  constexpr int LPR = HD / 4;  // lanes a row
+  const uint32_t row = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+  if (row >= n_rows) return;
+  const uint32_t tok = row / a.n_heads, head = row - tok * a.n_heads;
+  const uint32_t b = tok / a.q_len, qi = tok - b * a.q_len;
+  const uint32_t ctx = min(a.read_num[b], a.max_blocks << a.bs_log2);
+  const uint32_t r = qi * a.group + head % a.group;
+  const uint32_t np =
+      tile_keys_of<block_rows<HD, WAVES>(), tile_keys<HD, WAVES>()>(
+          a, a.pos_offset[b], ctx, r / block_rows<HD, WAVES>(), a.rows)
+          .pieces(a.split_keys);
+  if (np < 2) return;
+  const float2 *ml = reinterpret_cast<const float2 *>(a.ws_ml) + row;
+  const size_t at = (size_t)row * HD + (threadIdx.x % LPR) * 4;
+  const float *accp = a.ws_acc + at;
+  const size_t step = (size_t)n_rows * HD;
+  float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+  float M = kNegBig, L = 0.f;
+  for (uint32_t i = 0; i < np; i += 8) {
+    float2 x[8];
+    float4 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {  // (the last piece again past the end)
+      const uint32_t p = min(i + k, np - 1u);
+      x[k] = ml[(size_t)p * n_rows];
+      v[k] = *reinterpret_cast<const float4 *>(accp + p * step);
+    }
+    float mx = M;
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (x[k].y > 0.f) mx = fmaxf(mx, x[k].x);
+    const float corr = __builtin_amdgcn_exp2f(M - mx);
+    M = mx;
+    L *= corr;
+    acc.x *= corr;
+    acc.y *= corr;
+    acc.z *= corr;
+    acc.w *= corr;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      // (l = 0: the row sees no key of the piece)
+      const float w = i + k < np && x[k].y > 0.f
+                          ? __builtin_amdgcn_exp2f(x[k].x - M)
+                          : 0.f;
+      L += x[k].y * w;
+      acc.x += v[k].x * w;
+      acc.y += v[k].y * w;
+      acc.z += v[k].z * w;
+      acc.w += v[k].w * w;
+    }
+  }
+  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  *reinterpret_cast<float4 *>(a.out + at) =
+      make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
+}
+
+template <int HD, int WAVES, bool CUT>
+void launch_tiles(const PrefillArgs &a, dim3 grid, hipStream_t st) {
   // Past 64 KiB (head_dim 128 and 256 double-buffered) the dynamic LDS size
   // is declared to the runtime, once per instantiation and device.
   if constexpr (Lds<HD, WAVES>::bytes > 65536) {
@@ -1138,14 +1251,71 @@ void launch_prefill(const PrefillArgs &a, dim3 grid, hipStream_t st) {
         !(done.load(std::memory_order_relaxed) >> dev & 1u)) {
       // (a refusal shows as the launch's own error)
       if (hipFuncSetAttribute(
-              reinterpret_cast<const void *>(&prefill_kernel<HD, WAVES>),
+              reinterpret_cast<const void *>(&prefill_kernel<HD, WAVES, 1, CUT>),
               hipFuncAttributeMaxDynamicSharedMemorySize,
               (int)Lds<HD, WAVES>::bytes) == hipSuccess)
         done.fetch_or(1ull << dev, std::memory_order_relaxed);
     }
   }
-  hipLaunchKernelGGL((prefill_kernel<HD, WAVES>), grid, dim3(64 * WAVES),
-                     (Lds<HD, WAVES>::bytes), st, a);
+  hipLaunchKernelGGL((prefill_kernel<HD, WAVES, 1, CUT>), grid,
+                     dim3(64 * WAVES), (Lds<HD, WAVES>::bytes), st, a);
+}
+
+template <int HD, int WAVES>
+void launch_prefill(const PrefillArgs &a, dim3 grid, hipStream_t st) {
+  if (!a.split_keys) {
+    launch_tiles<HD, WAVES, false>(a, grid, st);
+    return;
+  }
+  launch_tiles<HD, WAVES, true>(a, dim3(grid.x * a.split_n), st);
+  const uint32_t n_rows = a.batch * a.q_len * a.n_heads;
+  constexpr uint32_t per = 256 / (HD / 4);
+  hipLaunchKernelGGL((prefill_reduce_kernel<HD, WAVES>),
+                     dim3((n_rows + per - 1) / per), dim3(256), 0, st, a,
+                     n_rows);
+}
+
+// Cuts the key ranges of a prefill whose query tiles leave the chip idle (a
+// short chunk behind a long context, a prompt on few KV heads): a workgroup
+// alone on its CU takes ~1 us a key tile whatever the others do, so the keys
+// are dealt out until the chip is one generation full. A kernel a layer:
+// Llama-3.2-1B heads, 300 rows behind 7700 keys (80 tiles) 123.6 -> 44.0 us
+// + 5.6 us for the reduction (35 us is this loop's rate on a full chip);
+// gemma-3 heads, 1000 rows, window 512 (32 tiles) 41.2 -> 24.1 + 5.3 us;
+// Qwen3-0.6B heads, 40 rows behind 6000 keys (8 tiles) 140 -> 19 us in all.
+// Pieces of at least four key tiles: at two the partials' traffic takes the
+// gain back (that Qwen3 call 26.0 against 28.7 us with prep). Cut only if
+// eight key tiles fewer remain: the reduction costs ~5 us, and Llama heads,
+// one prompt of 900 rows (232 tiles), lose 3.5 us a layer by it.
+void split_prefill(rvkv_pool *pool, PrefillArgs &a, uint32_t n_wg) {
+  const uint32_t hd = pool->head_dim;
+  const uint32_t bn = hd >= 256 ? 32 : 64;
+  // Workgroups resident at once.
+  const uint32_t want = 256u * (hd <= 64 ? 3 : hd == 128 ? 2 : 1);
+  if (n_wg >= want) return;
+  // The most keys a tile sees (the table bounds the context; the window the
+  // rest), and their average: a table as long as the chunk is a whole prompt.
+  const uint64_t cap = (uint64_t)a.max_blocks << a.bs_log2;
+  const uint64_t span =
+      a.window > 0 ? std::min<uint64_t>(
+                         cap, (uint64_t)a.window + 256 / a.group + 1 + bn)
+                   : cap;
+  const uint64_t avg =
+      a.window > 0 ? span : cap - std::min<uint64_t>(a.q_len, cap) / 2;
+  uint64_t keys = (avg * n_wg + want - 1) / want;
+  keys = std::max<uint64_t>((keys + bn - 1) / bn * bn, 4 * bn);
+  const uint64_t n_rows = (uint64_t)a.batch * a.q_len * a.n_heads;
+  const uint64_t most = kSplitBytes / (n_rows * (hd + 2) * 4);
+  if (most < 2) return;
+  if ((span + keys - 1) / keys > most)
+    keys = ((span + most - 1) / most + bn - 1) / bn * bn;
+  if (keys + 8 * bn > span) return;
+  void *ws = rvkv_detail::split_scratch(pool);
+  if (!ws) return;
+  a.split_keys = (uint32_t)keys;
+  a.split_n = (uint32_t)((span + keys - 1) / keys);
+  a.ws_acc = static_cast<float *>(ws);
+  a.ws_ml = a.ws_acc + (size_t)a.split_n * n_rows * hd;
 }
 
 // Waves per workgroup: 4 at head_dim 128 with the tiles staged by LDS DMA,
@@ -1234,6 +1404,7 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
   const uint64_t n_wg = (uint64_t)a.n_tiles * pool->n_kv * batch;
   if (n_wg > 0x7fffffffull)
     return fail(RVKV_EUNSUPPORTED, op, "too many query tiles for one launch");
+  split_prefill(pool, a, (uint32_t)n_wg);
   const dim3 grid((uint32_t)n_wg);
   switch (hd) {
     case 32: launch_prefill<32, 4>(a, grid, pool->stream); break;

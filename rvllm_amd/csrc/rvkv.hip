@@ -36,6 +36,21 @@ int hip_fail(const char *op, hipError_t e) {
   g_last_error = std::string(op) + ": " + hipGetErrorString(e);
   return RVKV_EHIP;
 }
+
+void *split_scratch(rvkv_pool *pool) {
+  if (!pool->split_base) return nullptr;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(pool->stream, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  if (cs != hipStreamCaptureStatusNone) return nullptr;
+  uint32_t i = 0;
+  while (i < pool->n_split && pool->split_stream[i] != pool->stream) ++i;
+  if (i == kSplitStreams) return nullptr;
+  if (i == pool->n_split) pool->split_stream[pool->n_split++] = pool->stream;
+  return pool->split_base + i * kSplitBytes;
+}
 }  // namespace rvkv_detail
 
 using rvkv_detail::fail;
@@ -1938,7 +1953,15 @@ int rvkv_pool_create(uint32_t n_layers, uint32_t num_blocks,
     return hip_fail(op, e);
   }
   const size_t bytes = p->tensor16 * 2 * 2 * n_layers;
-  e = hipMalloc(&p->base, bytes);
+  const size_t at = (bytes + 255) & ~(size_t)255;
+  e = hipMalloc(&p->base, at + rvkv_detail::kSplitStreams *
+                                   rvkv_detail::kSplitBytes);
+  if (e == hipSuccess) {
+    p->split_base = reinterpret_cast<unsigned char *>(p->base) + at;
+  } else {  // no room for the scratch regions: the cache alone
+    (void)hipGetLastError();
+    e = hipMalloc(&p->base, bytes);
+  }
   if (e != hipSuccess) {
     delete p;
     (void)hipGetLastError();

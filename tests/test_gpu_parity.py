@@ -1702,6 +1702,107 @@ def test_prefill_large_scores(hd):
     assert np.isfinite(out).all() and np.abs(out - want).max() < ATOL
 
 
+def _prefill_f64(st, q, tables, prior, read, window):
+    """Prefill attention in float64 from the raw cache (keys behind an
+    out-of-range id hidden), on the GPU."""
+    B, Q, H, hd = q.shape
+    nkv, bs = st.n_kv_heads, st.block_size
+    ids = dev_u32(np.arange(st.num_blocks))
+    kc, vc = (st.read_blocks(0, w, ids).double() for w in (0, 1))
+    out = torch.zeros(B, Q, H, hd, dtype=torch.float64, device="cuda")
+    for b in range(B):
+        t = torch.from_numpy(tables[b].astype(np.int64)).cuda()
+        ok = (t < st.num_blocks).repeat_interleave(bs)
+        t = t.clamp(max=st.num_blocks - 1)
+        k, v = (x[t].reshape(-1, nkv, hd) for x in (kc, vc))
+        j = torch.arange(k.shape[0], device="cuda")[None]
+        p = (int(prior[b]) + torch.arange(Q, device="cuda"))[:, None]
+        see = ok[None] & (j <= p) & (j < int(read[b]))
+        if window:
+            see &= j + window > p
+        for h in range(H):
+            s = q[b, :, h].double() @ k[:, h // (H // nkv)].T / hd ** 0.5
+            s = s.masked_fill(~see, -torch.inf)
+            w = torch.nan_to_num(torch.softmax(s, -1))
+            out[b, :, h] = w @ v[:, h // (H // nkv)]
+    return out
+
+
+@pytest.mark.parametrize("G,hd,bs,Q,prior,window", [
+    (4, 64, 16, 33, [2500, 700, 0], 0),   # pieces, one piece, a short prompt
+    (1, 64, 128, 3, [3000, 1], 0),
+    (3, 32, 8, 50, [1500, 64], 0),
+    (2, 128, 16, 1, [4095], 0),           # one row; a whole last piece
+    (2, 128, 16, 70, [1029, 1500], 900),
+    (4, 256, 16, 40, [1000, 37], 0),
+    (7, 256, 16, 200, [2000, 0], 700),    # two and more tiles a head
+])
+def test_prefill_cut_keys(G, hd, bs, Q, prior, window):
+    """Small grids over long contexts, whose keys are cut into pieces: every
+    number of pieces a tile, an out-of-range id inside a piece, and (under
+    graph capture) the same call uncut."""
+    rng = np.random.default_rng(hd + Q)
+    nkv, prior = 2, np.asarray(prior)
+    B, read = len(prior), prior + Q
+    mb = -(-int(read.max()) // bs)
+    st = HipKvStorage(1, B * mb + 3, bs, nkv, hd)
+    fill_layer(st, 0, seed=hd)
+    tables = rng.permutation(B * mb + 3)[:B * mb].reshape(B, mb).astype(
+        np.uint32)
+    q = torch.randn(B, Q, nkv * G, hd, device="cuda")
+    t, p, r = dev_u32(tables), dev_u32(prior), dev_u32(read)
+    out = st.paged_prefill(0, q, t, p, r, window=window)
+    want = _prefill_f64(st, q, tables, prior, read, window)
+    assert (out - want).abs().max() < ATOL
+    for _ in range(3):
+        assert torch.equal(st.paged_prefill(0, q, t, p, r, window=window),
+                           out)
+    # Captured: the keys are not cut.
+    outg = torch.empty_like(out)
+    graph = torch.cuda.CUDAGraph()
+    own = st.stream
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        st.set_stream(torch.cuda.current_stream())
+        st.paged_prefill(0, q, t, p, r, out=outg, window=window)
+    st.set_stream(own)
+    for _ in range(2):
+        outg.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert (outg - want).abs().max() < ATOL
+        assert torch.equal(st.paged_prefill(0, q, t, p, r, window=window),
+                           out)
+    # An unreadable block in the middle of the first sequence's context.
+    bad = tables.copy()
+    bad[0, (int(read[0]) // 2) // bs] = st.num_blocks + 5
+    out = st.paged_prefill(0, q, dev_u32(bad), p, r, window=window)
+    want = _prefill_f64(st, q, bad, prior, read, window)
+    assert (out - want).abs().max() < ATOL
+
+
+def test_prefill_cut_keys_streams():
+    """Calls queued on three streams at once: the first two get a scratch
+    region each, the third runs uncut; none disturbs another's partials."""
+    st = HipKvStorage(1, 260, 16, 2, 64)
+    fill_layer(st, 0, seed=9)
+    table = np.random.default_rng(9).permutation(260)[:256].astype(np.uint32)
+    t, p, r = dev_u32(table[None]), dev_u32([4000]), dev_u32([4040])
+    qs = [torch.randn(1, 40, 8, 64, device="cuda") for _ in range(3)]
+    want = [_prefill_f64(st, q, table[None], [4000], [4040], 0) for q in qs]
+    outs = [torch.empty_like(q) for q in qs]
+    own, streams = st.stream, [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for q, o, s in zip(qs, outs, streams):
+            st.set_stream(s)
+            st.paged_prefill(0, q, t, p, r, out=o)
+    torch.cuda.synchronize()
+    st.set_stream(own)
+    for o, w in zip(outs, want):
+        assert (o - w).abs().max() < ATOL
+
+
 def test_prefill_full_prompt_from_empty():
     """Whole-prompt prefill (pos_offset 0, read_num = q_len), the
     reference's first forward of a sequence, at 1000 tokens."""

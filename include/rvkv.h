@@ -304,10 +304,11 @@ int rvkv_attn_prep(rvkv_pool *pool, uint32_t layer, const float *q_in,
  * token-major [batch * q_len, n_heads, head_dim] f32, 16-byte aligned;
  * block_tables [batch, max_blocks] u32; pos_offset, read_num_tokens [batch]
  * u32 (all device). Table entries >= num_blocks mark keys unreadable (they
- * get probability 0); a row that sees no key gets zeros. With an f16 pool,
- * head_dim in {32, 64, 128, 256} and block_size a power of two >= 8 it is
- * computed on the matrix cores in f16 with f32 accumulation; any other
- * head_dim <= 1024, block size or an f32 pool runs a generic kernel in f32
+ * get probability 0); a row that sees no key gets zeros. At head_dim 32, 64,
+ * 128 or 256 and a power-of-two block_size it is computed on the matrix
+ * cores: in f16 with f32 accumulation over an f16 pool (block_size >= 8), in
+ * f32 over an f32 pool (block_size >= 4). Any other head_dim <= 1024 or block
+ * size runs a generic kernel in f32
  * arithmetic. Allocates nothing. Calls whose query rows alone leave the GPU
  * idle are cut along the keys and merged by a second launch; the partial
  * results go to the pool's scratch, half of which the first two streams that

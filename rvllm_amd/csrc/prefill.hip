@@ -291,6 +291,38 @@ __device__ __forceinline__ KeyRange tile_keys_of(const PrefillArgs &a,
           min(ctx, off + r1 / a.group + 1u)};
 }
 
+// The work of a prefill workgroup. XCD-aware order: workgroups are dispatched
+// round-robin over the 8 XCDs (each with its own L2), so workgroup w runs on
+// XCD w % 8. Renumber so each XCD gets a contiguous range of logical ids, in
+// which the query tiles of one (sequence, KV head) are adjacent: they re-read
+// the same K/V, which then stays in that XCD's L2. Within a head, long (late)
+// rows go first.
+struct WorkItem {
+  uint32_t tile, piece, kvh, b;
+};
+template <bool CUT>
+__device__ __forceinline__ WorkItem prefill_item(const PrefillArgs &a) {
+  const uint32_t n_wg = gridDim.x;
+  const uint32_t w = blockIdx.x, xcd = w % 8, idx = w / 8;
+  const uint32_t per = n_wg / 8, rem = n_wg % 8;
+  uint32_t logical = xcd < rem ? xcd * (per + 1) + idx
+                               : rem * (per + 1) + (xcd - rem) * per + idx;
+  // (Pieces: a causal prompt's late pieces hold fewer tiles, so a head
+  // spread over several XCDs goes round robin.)
+  if (CUT && (a.n_kv * a.batch) % 8 != 0) logical = w;
+  WorkItem i;
+  i.tile = a.n_tiles - 1 - logical % a.n_tiles;
+  uint32_t rest = logical / a.n_tiles;
+  i.piece = 0;
+  if (CUT) {  // the tiles of one piece re-read the same K/V
+    i.piece = rest % a.split_n;
+    rest /= a.split_n;
+  }
+  i.kvh = rest % a.n_kv;
+  i.b = rest / a.n_kv;
+  return i;
+}
+
 // WAVES wave64s per workgroup (4 or 8, 32 query rows each); the K/V tile
 // loads and LDS stores are shared among them, so more waves halve each
 // wave's share of that work. Registers are bounded for 8 resident waves per
@@ -354,12 +386,6 @@ __global__ void __launch_bounds__(
       return __syncthreads_or(x) != 0;
   };
 
-  // XCD-aware order: workgroups are dispatched round-robin over the 8 XCDs
-  // (each with its own L2), so workgroup w runs on XCD w % 8. Renumber so
-  // each XCD gets a contiguous range of logical ids, in which the query
-  // tiles of one (sequence, KV head) are adjacent: they re-read the same
-  // K/V, which then stays in that XCD's L2. Within a head, long (late)
-  // rows go first.
   uint32_t tile, kvh, b, item_lo = 0, item_hi = 0xFFFFFFFFu, slot = kNoSlot;
   uint32_t piece = 0;  // of a prefill tile's keys (a.split_keys)
   // Group item: member list (n, sequences, slots); its first member's
@@ -400,23 +426,11 @@ __global__ void __launch_bounds__(
     }
     tile = 0;
   } else {
-    const uint32_t n_wg = gridDim.x;
-    const uint32_t w = blockIdx.x, xcd = w % 8, idx = w / 8;
-    const uint32_t per = n_wg / 8, rem = n_wg % 8;
-    uint32_t logical =
-        xcd < rem ? xcd * (per + 1) + idx
-                  : rem * (per + 1) + (xcd - rem) * per + idx;
-    // (Pieces: a causal prompt's late pieces hold fewer tiles, so a head
-    // spread over several XCDs goes round robin.)
-    if (CUT && (a.n_kv * a.batch) % 8 != 0) logical = w;
-    tile = a.n_tiles - 1 - logical % a.n_tiles;
-    uint32_t rest = logical / a.n_tiles;
-    if (CUT) {  // the tiles of one piece re-read the same K/V
-      piece = rest % a.split_n;
-      rest /= a.split_n;
-    }
-    kvh = rest % a.n_kv;
-    b = rest / a.n_kv;
+    const WorkItem wi = prefill_item<CUT>(a);
+    tile = wi.tile;
+    piece = wi.piece;
+    kvh = wi.kvh;
+    b = wi.b;
   }
   const int tid = KSPLIT > 1 ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1176,12 +1190,378 @@ __global__ void __launch_bounds__(
   }
 }
 
-// Merges the pieces of the query tiles that prefill_kernel cut: HD / 4 lanes
+// Prefill over f32 cells, in f32 throughout (v_mfma_f32_32x32x2_f32: f32
+// products, f32 sums). One workgroup = (sequence, KV head, 32 query rows):
+// its four waves hold the same rows and take a quarter of the keys each,
+// merged through LDS at the end. Matrix layout as in prefill_kernel, S^T =
+// K . Q^T and O^T = V^T . P^T, with two dims or keys a step:
+//   S: step (i, e) contracts dims 8i + e and 8i + 4 + e, so a lane (key l %
+//      32, half h) feeds it from the float4 K[key][8i + 4h ..];
+//   P.V: step j contracts keys 8(j/4) + j%4 and that + 4, which is what
+//      accumulator register j holds in the two lane halves, so P feeds it
+//      from registers; the lane's rows of V^T are dims (l % 32) * DT + dt,
+//      DT consecutive floats of the key's row.
+// So no operand needs a shuffle, and K and V come straight from memory into
+// the operand registers: at 64 cycles a step the matrix cores take 4096
+// cycles for a 16 KiB tile (head_dim 64), so staging it in LDS for several
+// waves would save loads that nothing waits for. The next tile's K loads go
+// out behind the S product and its V loads behind P.V, into the registers
+// just read. Bound by the matrix cores (53 % busy; the rest is each wave's
+// ~6 us of start-up and merge and the last, partly filled generation).
+// Against one wave a (query head, row) in plain FMAs: SmolLM2 heads, one
+// prompt of 700 rows 777 -> 31 us a layer; Llama-3.2-1B heads, 1500 rows
+// 118 us (78 TFLOP/s). One, two or four waves a row tile: 700 rows 61, 44,
+// 31 us, 1500 rows 187, 125, 118 us. At three waves a SIMD (168 registers)
+// it spills: 155 us; two S chains instead of one: 119 us.
+constexpr int kF32Rows = 32, kF32Keys = 32, kF32Waves = 4;
+// At head_dim 256 the registers hold O and one of K and V: Q is in LDS, and
+// each tile's K and V are loaded when they are needed.
+template <int HD>
+constexpr bool kF32Ahead = HD <= 128;
+template <int HD>
+constexpr size_t kF32QBytes = kF32Ahead<HD> ? 0 : (size_t)kF32Rows * HD * 4;
+template <int HD>
+constexpr size_t kF32LdsBytes =
+    kF32QBytes<HD> + (size_t)kF32Waves * kF32Keys * kF32Rows * 4 +
+    (size_t)(kF32Waves - 1) * (2 + HD / 32 * 16) * 64 * 4;
+
+template <int HD, bool CUT>
+__global__ void __launch_bounds__(64 * kF32Waves, HD <= 64 ? 2 : 1)
+    prefill_f32_kernel(PrefillArgs a) {
+  constexpr int BN = kF32Keys, KI = HD / 8, DT = HD / 32;
+  constexpr bool AHEAD = kF32Ahead<HD>;
+  extern __shared__ __align__(16) unsigned char smem_f32[];
+  float4 *q_s = reinterpret_cast<float4 *>(smem_f32);
+  float *rowp_s = reinterpret_cast<float *>(smem_f32 + kF32QBytes<HD>);
+  float *merge_s = rowp_s + kF32Waves * kF32Keys * kF32Rows;
+  const WorkItem wi = prefill_item<CUT>(a);
+  const uint32_t b = wi.b, kvh = wi.kvh;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, hl = lane >> 5, ln = lane & 31;
+  typedef const __attribute__((address_space(4))) uint32_t cu32;
+  const uint32_t ctx = min(*(cu32 *)(uintptr_t)(a.read_num + b),
+                           a.max_blocks << a.bs_log2);
+  const uint32_t off = *(cu32 *)(uintptr_t)(a.pos_offset + b);
+  const uint32_t *table = a.tables + (size_t)b * a.max_blocks;
+  const uint32_t bs_mask = (1u << a.bs_log2) - 1u;
+
+  const KeyRange kr = tile_keys_of<kF32Rows, BN>(a, off, ctx, wi.tile, a.rows);
+  uint32_t lo = kr.begin, hi = max(kr.end, kr.begin);
+  bool partial = false;
+  if constexpr (CUT) {
+    const uint32_t np = kr.pieces(a.split_keys);
+    if (wi.piece >= np && wi.piece > 0) return;  // (the reduction skips it)
+    partial = np > 1;
+    lo += wi.piece * a.split_keys;
+    hi = min(hi, lo + a.split_keys);
+  }
+  // This wave's share, in whole tiles.
+  {
+    const uint32_t nt = (hi - lo + BN - 1) / BN;
+    const uint32_t sub = (nt + kF32Waves - 1) / kF32Waves * BN;
+    lo = min(lo + wave * sub, hi);
+    hi = min(lo + sub, hi);
+  }
+
+  // This lane's query row, and the keys that every row sees.
+  const uint32_t r0 = wi.tile * kF32Rows, r = r0 + ln;
+  const uint32_t r1 = min(r0 + kF32Rows, a.rows) - 1u;
+  const bool row_ok = r < a.rows;
+  const uint32_t qi = row_ok ? r / a.group : 0u;
+  const uint32_t head = kvh * a.group + (row_ok ? r - qi * a.group : 0u);
+  const uint32_t row_hi = row_ok ? min(hi, off + qi + 1u) : 0u;
+  const uint32_t row_lo = lo_bound(off + qi, a.window);
+  const uint32_t all_hi = min(hi, off + r0 / a.group + 1u);
+  const uint32_t all_lo = lo_bound(off + r1 / a.group, a.window);
+  const size_t qrow = ((size_t)b * a.q_len + qi) * a.n_heads + head;
+
+  float4 q[AHEAD ? KI : 1];
+  auto read_q = [&](int i) {
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (row_ok)
+      x = *reinterpret_cast<const float4 *>(a.q + qrow * HD + 8 * i + 4 * hl);
+    return make_float4(x.x * a.qscale, x.y * a.qscale, x.z * a.qscale,
+                       x.w * a.qscale);
+  };
+  if constexpr (AHEAD) {
+#pragma unroll
+    for (int i = 0; i < KI; ++i) q[i] = read_q(i);
+  } else {  // (the waves hold the same rows in the same lanes)
+#pragma unroll
+    for (int i = 0; i < KI / kF32Waves; ++i)
+      q_s[(i * kF32Waves + wave) * 64 + lane] = read_q(i * kF32Waves + wave);
+    __syncthreads();
+  }
+  f32x16 o[DT];
+#pragma unroll
+  for (int t = 0; t < DT; ++t)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[t][j] = 0.f;
+  float m = kNegBig, l = 0.f;
+
+  const char *kbase =
+      reinterpret_cast<const char *>(a.kc) + (size_t)kvh * a.head_stride * 4;
+  const char *vbase =
+      reinterpret_cast<const char *>(a.vc) + (size_t)kvh * a.head_stride * 4;
+  const uint64_t blk_bytes = a.block_stride * 4;
+
+  // Block ids of a tile's eight groups of four keys (a block holds at least
+  // four), by scalar loads: vector loads would wait behind the K/V loads in
+  // flight.
+  cu32 *ctable = (cu32 *)(uintptr_t)table;
+  auto fetch_ids = [&](uint32_t (&ids)[8], uint32_t kt) {
+#pragma unroll
+    for (int g = 0; g < 8; ++g)
+      ids[g] = ctable[min((kt + 4 * g) >> a.bs_log2, a.max_blocks - 1u)];
+  };
+  float4 kf[KI];
+  float vf[16][DT];
+  // (an unreadable block's keys load block 0: masked, and their V zeroed)
+  auto load_k = [&](const uint32_t (&ids)[8], uint32_t kt) {
+    // the id of key kt + ln (values first: a select between array elements
+    // would keep the array in memory)
+    const uint32_t i0 = ids[0], i1 = ids[1], i2 = ids[2], i3 = ids[3],
+                   i4 = ids[4], i5 = ids[5], i6 = ids[6], i7 = ids[7];
+    const uint32_t a0 = ln & 4 ? i1 : i0, a1 = ln & 4 ? i3 : i2;
+    const uint32_t a2 = ln & 4 ? i5 : i4, a3 = ln & 4 ? i7 : i6;
+    const uint32_t b0 = ln & 8 ? a1 : a0, b1 = ln & 8 ? a3 : a2;
+    const uint32_t id = ln & 16 ? b1 : b0;
+    const char *p = kbase + (id < a.num_blocks ? id : 0u) * blk_bytes +
+                    ((kt + ln) & bs_mask) * (HD * 4) + 16 * hl;
+#pragma unroll
+    for (int i = 0; i < KI; ++i)
+      kf[i] = *reinterpret_cast<const float4 *>(p + 32 * i);
+  };
+  auto load_v = [&](const uint32_t (&ids)[8], uint32_t kt) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const uint32_t i0 = ids[2 * g], i1 = ids[2 * g + 1];
+      const uint32_t ig = hl ? i1 : i0;
+      const char *p = vbase + (ig < a.num_blocks ? ig : 0u) * blk_bytes +
+                      ((kt + 8 * g + 4 * hl) & bs_mask) * (HD * 4) +
+                      ln * (DT * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float *x = reinterpret_cast<const float *>(p + e * (HD * 4));
+        if constexpr (DT == 1) {
+          vf[4 * g + e][0] = x[0];
+        } else if constexpr (DT == 2) {
+          const float2 y = *reinterpret_cast<const float2 *>(x);
+          vf[4 * g + e][0] = y.x;
+          vf[4 * g + e][1] = y.y;
+        } else {
+#pragma unroll
+          for (int t = 0; t < DT; t += 4) {
+            const float4 y = *reinterpret_cast<const float4 *>(x + t);
+            vf[4 * g + e][t] = y.x;
+            vf[4 * g + e][t + 1] = y.y;
+            vf[4 * g + e][t + 2] = y.z;
+            vf[4 * g + e][t + 3] = y.w;
+          }
+        }
+      }
+    }
+  };
+
+  uint32_t id[8], id_next[8];
+  if (lo < hi) {
+    fetch_ids(id, lo);
+    if constexpr (AHEAD) {
+      load_k(id, lo);
+      load_v(id, lo);
+    }
+    fetch_ids(id_next, lo + BN);
+  }
+  for (uint32_t kt = lo; kt < hi; kt += BN) {
+    uint32_t bad = 0;  // keys behind unreadable blocks
+#pragma unroll
+    for (int g = 0; g < 8; ++g)
+      bad |= id[g] < a.num_blocks ? 0u : 0xFu << (4 * g);
+    if constexpr (!AHEAD) load_k(id, kt);
+    f32x16 s;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) s[j] = 0.f;
+#pragma unroll
+    for (int i = 0; i < KI; ++i) {
+      const float4 qi4 = AHEAD ? q[AHEAD ? i : 0] : q_s[i * 64 + lane];
+      const float k4[4] = {kf[i].x, kf[i].y, kf[i].z, kf[i].w};
+      const float q4[4] = {qi4.x, qi4.y, qi4.z, qi4.w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4[e], q4[e], s, 0, 0, 0);
+    }
+    // (Past the last tile, that tile again: with loads on one path only, the
+    // compiler's waits count exactly.)
+    const bool more = kt + BN < hi;
+    const uint32_t kn = more ? kt + BN : kt;
+    uint32_t id_n[8];
+#pragma unroll
+    for (int g = 0; g < 8; ++g) {
+      const uint32_t x = id_next[g], y = id[g];
+      id_n[g] = more ? x : y;
+    }
+    if constexpr (AHEAD) {
+      load_k(id_n, kn);
+    } else {  // (not before K's registers are free)
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(id, kt);
+    }
+
+    const bool whole = bad == 0 && kt >= all_lo && kt + BN <= all_hi;
+    if (!whole) {
+      const uint32_t c = 4 * hl;  // register j: key kt + c + 8 (j/4) + j%4
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const uint32_t kk = c + 8 * (j / 4) + j % 4;
+        const bool ok = kt + kk >= row_lo && kt + kk < row_hi &&
+                        !((bad >> kk) & 1u);
+        s[j] = ok ? s[j] : -__builtin_inff();
+        if (kt + kk >= hi || ((bad >> kk) & 1u)) {  // never read
+#pragma unroll
+          for (int t = 0; t < DT; ++t) vf[j][t] = 0.f;
+        }
+      }
+    }
+    float mx = m;
+#pragma unroll
+    for (int j = 0; j < 16; j += 2) mx = vmax3(mx, s[j], s[j + 1]);
+    mx = max_halves(mx);
+    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
+      const float alpha = __builtin_amdgcn_exp2f(m - mx);
+      m = mx;
+      l *= alpha;
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) o[t][j] *= alpha;
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      s[j] = __builtin_amdgcn_exp2f(s[j] - m);
+      l += s[j];
+    }
+    // In a tile that some rows see only in part, a V that is not finite must
+    // not meet another row's zero weight (0 * inf): it is left out of the
+    // product and added row by row afterwards.
+    bool by_row = false;
+    if (!whole) {
+      bool odd = false;
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+#pragma unroll
+        for (int t = 0; t < DT; ++t)
+          odd |= !(__builtin_fabsf(vf[j][t]) < __builtin_inff());
+      by_row = __builtin_amdgcn_ballot_w64(odd) != 0;
+      if (by_row) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+#pragma unroll
+          for (int t = 0; t < DT; ++t)
+            vf[j][t] = __builtin_fabsf(vf[j][t]) < __builtin_inff() ? vf[j][t]
+                                                                    : 0.f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+        o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(vf[j][t], s[j], o[t], 0, 0,
+                                                    0);
+    if (by_row) {
+      float *p_s = rowp_s + wave * (BN * 32);  // [key][row] of this wave
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        p_s[(8 * (j / 4) + 4 * hl + j % 4) * 32 + ln] = s[j];
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 1
+      for (uint32_t kk = 0; kk < min(hi - kt, (uint32_t)BN); ++kk) {
+        const float pk = p_s[kk * 32 + ln];
+        const uint32_t bk =
+            table[min((kt + kk) >> a.bs_log2, a.max_blocks - 1u)];
+        const float *row = reinterpret_cast<const float *>(
+            vbase + (bk < a.num_blocks ? bk : 0u) * blk_bytes +
+            ((kt + kk) & bs_mask) * (HD * 4));
+#pragma unroll
+        for (int t = 0; t < DT; ++t) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float v = row[(8 * (i / 4) + 4 * hl + i % 4) * DT + t];
+            const bool add = pk != 0.f && !(__builtin_fabsf(v) < __builtin_inff());
+            o[t][i] = add ? __builtin_fmaf(pk, v, o[t][i]) : o[t][i];
+          }
+          __builtin_amdgcn_sched_barrier(0);  // (bounds the loads in flight)
+        }
+      }
+    }
+    if constexpr (AHEAD)
+      load_v(id_n, kn);
+    else
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int g = 0; g < 8; ++g) id[g] = id_n[g];
+    fetch_ids(id_next, kt + 2 * BN);
+  }
+
+  // Merge the waves' states into wave 0, lane-wise (the same rows in the
+  // same layout in every wave).
+  constexpr int NV = 2 + DT * 16;
+  l = sum_halves(l);
+  if (wave > 0) {
+    float *dst = merge_s + (size_t)(wave - 1) * NV * 64 + lane;
+    dst[0] = m;
+    dst[64] = l;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int j = 0; j < 16; ++j) dst[(2 + t * 16 + j) * 64] = o[t][j];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int w = 1; w < kF32Waves; ++w) {
+    const float *src = merge_s + (size_t)(w - 1) * NV * 64 + lane;
+    const float mw = src[0], lw = src[64];
+    const float M = fmaxf(m, mw);
+    const float aw = __builtin_amdgcn_exp2f(m - M);
+    const float bw = __builtin_amdgcn_exp2f(mw - M);
+    l = l * aw + lw * bw;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int j = 0; j < 16; ++j)
+        o[t][j] = o[t][j] * aw + src[(2 + t * 16 + j) * 64] * bw;
+    m = M;
+  }
+  if (!row_ok) return;
+  const size_t idx =
+      partial ? (size_t)wi.piece * a.batch * a.q_len * a.n_heads + qrow : qrow;
+  float *op = (partial ? a.ws_acc : a.out) + idx * HD;
+  const float inv = partial ? 1.f : (l > 0.f ? 1.0f / l : 0.f);
+#pragma unroll
+  for (int g = 0; g < 4; ++g)
+#pragma unroll
+    for (int f = 0; f < DT; ++f) {  // dims (8g + 4hl) * DT + 4f ..
+      float x[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        x[e] = o[(4 * f + e) % DT][4 * g + (4 * f + e) / DT] * inv;
+      *reinterpret_cast<float4 *>(op + (8 * g + 4 * hl) * DT + 4 * f) =
+          make_float4(x[0], x[1], x[2], x[3]);
+    }
+  if (partial && hl == 0) {
+    a.ws_ml[idx * 2] = m;
+    a.ws_ml[idx * 2 + 1] = l;
+  }
+}
+
+// Merges the pieces of the query tiles that the prefill kernels cut: HD / 4 lanes
 // of a q row (token, head), four elements each; weights 2^(m_i - M). Rows of
 // uncut tiles are left alone (the prefill kernel wrote them). Bound by the
 // launch and the round trips to the partials: eight pieces' (m, l) and
 // partials are loaded at a time.
-template <int HD, int WAVES>
+template <int HD, int BM, int BN>
 __global__ void __launch_bounds__(256)
     prefill_reduce_kernel(PrefillArgs a, uint32_t n_rows) {
   constexpr int LPR = HD / 4;  // lanes a row
@@ -1192,8 +1572,7 @@ __global__ void __launch_bounds__(256)
   const uint32_t ctx = min(a.read_num[b], a.max_blocks << a.bs_log2);
   const uint32_t r = qi * a.group + head % a.group;
   const uint32_t np =
-      tile_keys_of<block_rows<HD, WAVES>(), tile_keys<HD, WAVES>()>(
-          a, a.pos_offset[b], ctx, r / block_rows<HD, WAVES>(), a.rows)
+      tile_keys_of<BM, BN>(a, a.pos_offset[b], ctx, r / BM, a.rows)
           .pieces(a.split_keys);
   if (np < 2) return;
   const float2 *ml = reinterpret_cast<const float2 *>(a.ws_ml) + row;
@@ -1240,23 +1619,35 @@ __global__ void __launch_bounds__(256)
       make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
 }
 
+template <int HD, int BM, int BN>
+void launch_prefill_reduce(const PrefillArgs &a, hipStream_t st) {
+  const uint32_t n_rows = a.batch * a.q_len * a.n_heads;
+  constexpr uint32_t per = 256 / (HD / 4);
+  hipLaunchKernelGGL((prefill_reduce_kernel<HD, BM, BN>),
+                     dim3((n_rows + per - 1) / per), dim3(256), 0, st, a,
+                     n_rows);
+}
+
+// Past 64 KiB the dynamic LDS size is declared to the runtime, once per
+// kernel and device.
+template <auto Kernel>
+void declare_lds(size_t bytes) {
+  if (bytes <= 65536) return;
+  static std::atomic<uint64_t> done{0};
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev < 64 &&
+      !(done.load(std::memory_order_relaxed) >> dev & 1u)) {
+    // (a refusal shows as the launch's own error)
+    if (hipFuncSetAttribute(reinterpret_cast<const void *>(Kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)bytes) == hipSuccess)
+      done.fetch_or(1ull << dev, std::memory_order_relaxed);
+  }
+}
+
 template <int HD, int WAVES, bool CUT>
 void launch_tiles(const PrefillArgs &a, dim3 grid, hipStream_t st) {
-  // Past 64 KiB (head_dim 128 and 256 double-buffered) the dynamic LDS size
-  // is declared to the runtime, once per instantiation and device.
-  if constexpr (Lds<HD, WAVES>::bytes > 65536) {
-    static std::atomic<uint64_t> done{0};
-    int dev = 0;
-    if (hipGetDevice(&dev) == hipSuccess && dev < 64 &&
-        !(done.load(std::memory_order_relaxed) >> dev & 1u)) {
-      // (a refusal shows as the launch's own error)
-      if (hipFuncSetAttribute(
-              reinterpret_cast<const void *>(&prefill_kernel<HD, WAVES, 1, CUT>),
-              hipFuncAttributeMaxDynamicSharedMemorySize,
-              (int)Lds<HD, WAVES>::bytes) == hipSuccess)
-        done.fetch_or(1ull << dev, std::memory_order_relaxed);
-    }
-  }
+  declare_lds<&prefill_kernel<HD, WAVES, 1, CUT>>(Lds<HD, WAVES>::bytes);
   hipLaunchKernelGGL((prefill_kernel<HD, WAVES, 1, CUT>), grid,
                      dim3(64 * WAVES), (Lds<HD, WAVES>::bytes), st, a);
 }
@@ -1268,11 +1659,25 @@ void launch_prefill(const PrefillArgs &a, dim3 grid, hipStream_t st) {
     return;
   }
   launch_tiles<HD, WAVES, true>(a, dim3(grid.x * a.split_n), st);
-  const uint32_t n_rows = a.batch * a.q_len * a.n_heads;
-  constexpr uint32_t per = 256 / (HD / 4);
-  hipLaunchKernelGGL((prefill_reduce_kernel<HD, WAVES>),
-                     dim3((n_rows + per - 1) / per), dim3(256), 0, st, a,
-                     n_rows);
+  launch_prefill_reduce<HD, block_rows<HD, WAVES>(), tile_keys<HD, WAVES>()>(
+      a, st);
+}
+
+template <int HD, bool CUT>
+void launch_tiles_f32(const PrefillArgs &a, dim3 grid, hipStream_t st) {
+  declare_lds<&prefill_f32_kernel<HD, CUT>>(kF32LdsBytes<HD>);
+  hipLaunchKernelGGL((prefill_f32_kernel<HD, CUT>), grid,
+                     dim3(64 * kF32Waves), kF32LdsBytes<HD>, st, a);
+}
+
+template <int HD>
+void launch_prefill_f32(const PrefillArgs &a, dim3 grid, hipStream_t st) {
+  if (!a.split_keys) {
+    launch_tiles_f32<HD, false>(a, grid, st);
+    return;
+  }
+  launch_tiles_f32<HD, true>(a, dim3(grid.x * a.split_n), st);
+  launch_prefill_reduce<HD, kF32Rows, kF32Keys>(a, st);
 }
 
 // Cuts the key ranges of a prefill whose query tiles leave the chip idle (a
@@ -1289,9 +1694,13 @@ void launch_prefill(const PrefillArgs &a, dim3 grid, hipStream_t st) {
 // one prompt of 900 rows (232 tiles), lose 3.5 us a layer by it.
 void split_prefill(rvkv_pool *pool, PrefillArgs &a, uint32_t n_wg) {
   const uint32_t hd = pool->head_dim;
-  const uint32_t bn = hd >= 256 ? 32 : 64;
+  // (f32 cells: tiles of 32 keys, four at a time; their workgroups are cut
+  // until there is one a CU: at two, a prompt of 700 rows took 31 + 5 us
+  // against 31 us uncut)
+  const uint32_t bn = pool->f32() || hd >= 256 ? 32 : 64;
   // Workgroups resident at once.
-  const uint32_t want = 256u * (hd <= 64 ? 3 : hd == 128 ? 2 : 1);
+  const uint32_t want =
+      256u * (pool->f32() || hd >= 256 ? 1 : hd == 128 ? 2 : 3);
   if (n_wg >= want) return;
   // The most keys a tile sees (the table bounds the context; the window the
   // rest), and their average: a table as long as the chunk is a whole prompt.
@@ -1303,7 +1712,8 @@ void split_prefill(rvkv_pool *pool, PrefillArgs &a, uint32_t n_wg) {
   const uint64_t avg =
       a.window > 0 ? span : cap - std::min<uint64_t>(a.q_len, cap) / 2;
   uint64_t keys = (avg * n_wg + want - 1) / want;
-  keys = std::max<uint64_t>((keys + bn - 1) / bn * bn, 4 * bn);
+  keys = std::max<uint64_t>((keys + bn - 1) / bn * bn,
+                            pool->f32() ? 8 * bn : 4 * bn);
   const uint64_t n_rows = (uint64_t)a.batch * a.q_len * a.n_heads;
   const uint64_t most = kSplitBytes / (n_rows * (hd + 2) * 4);
   if (most < 2) return;
@@ -1360,13 +1770,15 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
     return fail(RVKV_EINVAL, op, "q and out must be 16-byte aligned");
   if (!(scale > 0.f) || !std::isfinite(scale))
     return fail(RVKV_EINVAL, op, "scale must be positive and finite");
-  // The matrix-core kernel takes f16 cells, head_dim 32/64/128/256 and
-  // power-of-two blocks of >= 8 tokens; every other shape (and an f32
-  // cache) runs the generic kernel.
-  if (pool->f32() || (hd != 32 && hd != 64 && hd != 128 && hd != 256) ||
-      bs < 8 || (bs & (bs - 1)) != 0 ||
+  // The matrix-core kernels take head_dim 32/64/128/256 and power-of-two
+  // blocks, of >= 8 tokens (f16 cells) or >= 4 (f32 cells, whose batch and
+  // q_len stay bounded as in the generic kernel); every other shape runs the
+  // generic kernel.
+  if ((hd != 32 && hd != 64 && hd != 128 && hd != 256) ||
+      bs < (pool->f32() ? 4u : 8u) || (bs & (bs - 1)) != 0 ||
       (uint64_t)max_blocks * bs > 0x80000000ull ||
-      pool->block_elems * 2 >= 0x100000000ull)
+      (pool->f32() ? batch > 65535 || q_len > 65535
+                   : pool->block_elems * 2 >= 0x100000000ull))
     return rvkv_detail::generic_attention(
         op, pool, layer, q, block_tables, max_blocks, pos_offset,
         read_num_tokens, batch, q_len, n_heads, 0xFFFFFFFFu, scale, window,
@@ -1395,7 +1807,9 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
   a.bs_log2 = lg;
   a.rows = (uint32_t)rows;
   const uint32_t waves = prefill_waves(hd);
-  const uint32_t bm = kWaveRows * (split_dims((int)hd) ? waves / 2 : waves);
+  const uint32_t bm =
+      pool->f32() ? kF32Rows
+                  : kWaveRows * (split_dims((int)hd) ? waves / 2 : waves);
   a.n_tiles = (uint32_t)((rows + bm - 1) / bm);
   a.qscale = scale * 1.4426950408889634f;
   a.window = window;
@@ -1406,6 +1820,16 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
     return fail(RVKV_EUNSUPPORTED, op, "too many query tiles for one launch");
   split_prefill(pool, a, (uint32_t)n_wg);
   const dim3 grid((uint32_t)n_wg);
+  if (pool->f32()) {
+    switch (hd) {
+      case 32: launch_prefill_f32<32>(a, grid, pool->stream); break;
+      case 64: launch_prefill_f32<64>(a, grid, pool->stream); break;
+      case 128: launch_prefill_f32<128>(a, grid, pool->stream); break;
+      default: launch_prefill_f32<256>(a, grid, pool->stream); break;
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? RVKV_OK : hip_fail(op, e);
+  }
   switch (hd) {
     case 32: launch_prefill<32, 4>(a, grid, pool->stream); break;
     case 64:

@@ -243,3 +243,67 @@ def test_f32_smollm2_config():
                           _bits(ref.v))
 
 
+
+
+@pytest.mark.parametrize("G,hd,bs,Q,prior,window", [
+    (3, 64, 16, 5, [0, 30], 0),          # less than one tile of rows or keys
+    (3, 64, 16, 32, [1, 2000], 0),       # pieces beside a short prompt
+    (1, 32, 4, 33, [0, 127, 96], 0),     # the smallest block, tile edges
+    (4, 32, 8, 70, [900], 300),
+    (2, 128, 16, 64, [64, 0], 0),
+    (2, 128, 32, 21, [1700], 1000),
+    (4, 256, 16, 40, [0, 700], 0),
+    (1, 256, 128, 100, [3], 40),
+    (5, 64, 16, 700, [0], 0),            # whole tiles seen by every row
+])
+def test_f32_prefill(G, hd, bs, Q, prior, window):
+    """Prefill on the f32 matrix cores against float64, with ragged read
+    counts, windows, cut keys and an out-of-range block id. Every product and
+    sum is f32: 2e-5, as for the reference's own f32 cases."""
+    from tests.test_gpu_parity import _prefill_f64
+    rng = np.random.default_rng(hd + Q)
+    nkv, prior = 2, np.asarray(prior)
+    B, read = len(prior), prior + Q
+    read[-1] = max(1, read[-1] - 2)
+    mb = -(-int((prior + Q).max()) // bs)
+    nb = B * mb + 3
+    st = HipKvStorage(1, nb, bs, nkv, hd, dtype=torch.float32)
+    at = torch.arange(nb * bs, device="cuda")
+    k, v = (torch.randn(nb * bs, nkv, hd, device="cuda") for _ in range(2))
+    st.write_tokens(0, (at // bs).int(), (at % bs).int(), k, v)
+    tables = rng.permutation(nb)[:B * mb].reshape(B, mb).astype(np.uint32)
+    q = torch.randn(B, Q, nkv * G, hd, device="cuda")
+    for bad in (None, (int(read[0]) // 2) // bs):
+        if bad is not None:
+            tables[0, bad] = nb + 9
+        t, p, r = dev_u32(tables), dev_u32(prior), dev_u32(read)
+        out = st.paged_prefill(0, q, t, p, r, window=window)
+        want = _prefill_f64(st, q, tables, prior, read, window)
+        assert (out - want).abs().max() < 2e-5
+        assert torch.equal(st.paged_prefill(0, q, t, p, r, window=window),
+                           out)
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
+def test_f32_prefill_inf_value(hd):
+    """A V row that is not finite reaches the rows that see it, and no
+    others, wherever it lies in a key tile."""
+    from tests.test_gpu_parity import _prefill_f64
+    Q, nb, bs = 100, 7, 16
+    table = np.random.default_rng(hd).permutation(nb).astype(np.uint32)
+    for key in (0, 37, 63, 64, 99):
+        st = HipKvStorage(1, nb, bs, 1, hd, dtype=torch.float32)
+        k, v = (torch.randn(Q, 1, hd, device="cuda") for _ in range(2))
+        at = np.arange(Q)
+        slots = dev_u32(table[at // bs]), dev_u32(at % bs)
+        st.write_tokens(0, *slots, k, v)
+        q = torch.randn(1, Q, 2, hd, device="cuda")
+        args = dev_u32(table[None]), dev_u32([0]), dev_u32([Q])
+        want = _prefill_f64(st, q, table[None], [0], [Q], 0)
+        v[key, 0, hd // 2] = float("inf")
+        st.write_tokens(0, *slots, k, v)
+        out = st.paged_prefill(0, q, *args)
+        assert torch.isfinite(out[0, :key]).all()
+        assert torch.isinf(out[0, key:, :, hd // 2]).all()
+        out[0, key:, :, hd // 2] = want[0, key:, :, hd // 2].float()
+        assert (out - want).abs().max() < 2e-5

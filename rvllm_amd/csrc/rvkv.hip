@@ -631,6 +631,8 @@ struct DecodeArgs {
   uint32_t max_tokens;
   // Host-side: the shape runs the generic kernel (generic.hip).
   uint32_t generic;
+  // Host-side: the most partitions a sequence is split into.
+  uint32_t max_parts;
 };
 
 constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
@@ -638,6 +640,13 @@ constexpr uint32_t kNoSlot = 0xFFFFFFFFu;
 // A plan item whose seq field has this bit is a shared-prefix group item
 // (matrix-core decode only); the other bits locate its member list.
 constexpr uint32_t kGroupItem = 0x80000000u;
+
+// Most waves a decode workgroup can have: what the kernel's registers leave
+// room for.
+constexpr int decode_max_waves(int hd, int gt, bool f32) {
+  return f32 ? (hd <= 128 ? (gt <= 7 ? 16 : 4) : (gt <= 4 ? 8 : 4))
+             : (gt <= 4 ? 8 : 4);
+}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp(float x) {
@@ -862,7 +871,8 @@ __device__ __forceinline__ void decode_chunk(SoftmaxState<GT, NL> &st,
 // normalised output; otherwise it writes its partial (m, l, acc) and the
 // reduction kernel merges the partitions.
 template <int HD, int GT, int U, int NL, bool RAGGED>
-__global__ void __launch_bounds__(256) decode_part_kernel(
+__global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, false))
+    decode_part_kernel(
     const uint4 *p_items, const uint32_t *p_tables, const uint32_t *p_ctx,
     uint32_t p_mb, uint32_t p_bs, uint32_t p_pt, DecodeArgs a) {
   // (The start-up chain's inputs come as leading arguments, which the
@@ -1280,7 +1290,11 @@ __global__ void __launch_bounds__(256) decode_part_kernel(
 // HD / (4 NL) lanes per row, RPL = 64 / R rows per wave-wide load. Masked
 // keys load zero rows, as in the f16 kernel.
 template <int HD, int GT>
-__global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
+__global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, true))
+    decode_f32_kernel(const uint4 *p_items, const uint32_t *p_tables,
+                      const uint32_t *p_ctx, uint32_t p_mb, uint32_t p_bs,
+                      uint32_t p_pt, DecodeArgs a) {
+  // (leading arguments as in decode_part_kernel)
   constexpr int NL = HD >= 256 ? 2 : 1;
   constexpr int R = HD / (4 * NL);
   constexpr int RPL = 64 / R;
@@ -1295,16 +1309,16 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
   const int rg = lane / R, c = lane % R;
   uint32_t b, t0, tend, slot;
   uint32_t hy = blockIdx.y;
-  if (a.items) {
-    const uint4 it = sload4(a.items + blockIdx.x);
+  if (p_items) {
+    const uint4 it = sload4(p_items + blockIdx.x);
     b = it.x;
     t0 = it.y;
     tend = it.z;
     slot = it.w;
   } else {
     b = blockIdx.z;
-    t0 = blockIdx.x * a.part_tokens;
-    tend = t0 + a.part_tokens;
+    t0 = blockIdx.x * p_pt;
+    tend = t0 + p_pt;
     slot = a.n_parts > 1 ? b * a.n_parts + blockIdx.x : kNoSlot;
     hy = (hy + b) % gridDim.y;  // (as in the f16 kernel: heads over XCDs)
   }
@@ -1313,7 +1327,15 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
   const uint32_t h0 = kvh * a.group + sub * GT;
   const uint32_t ng = min((uint32_t)GT, a.group - sub * GT);
   typedef const __attribute__((address_space(4))) uint32_t cu32;
-  cu32 *table = (cu32 *)(uintptr_t)(a.tables + (size_t)b * a.max_blocks);
+  cu32 *table = (cu32 *)(uintptr_t)(p_tables + (size_t)b * p_mb);
+  // The first block ids go out with the context length (clamped to the
+  // table for now).
+  const uint32_t first = t0 + (uint32_t)wave * TC;
+  const uint32_t mb1 = p_mb - 1;
+  uint32_t ids[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    ids[u] = table[min((first + u * RPL) >> p_bs, mb1)];
 
   float4 q[GT][NL];
 #pragma unroll
@@ -1327,11 +1349,11 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
                             x.w * a.qscale);
     }
   }
-  uint32_t ctx = min(sload(a.ctx_lens + b), a.ctx_cap);
+  uint32_t ctx = min(sload(p_ctx + b), a.ctx_cap);
   const uint32_t lo =
       (a.window > 0 && ctx > (uint32_t)a.window) ? ctx - (uint32_t)a.window : 0;
   const uint32_t t1 = min(tend, ctx);
-  if (!a.items && ctx <= a.part_tokens) slot = kNoSlot;
+  if (!p_items && ctx <= p_pt) slot = kNoSlot;
   if (t0 >= t1) {
     if (ctx == 0 && t0 == 0 && wave == 0 && rg == 0)
       for (uint32_t g = 0; g < ng; ++g)
@@ -1351,11 +1373,10 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
 #pragma unroll
     for (int e = 0; e < NL * 4; ++e) acc[g][e] = 0.f;
   }
-  const uint32_t first = t0 + (uint32_t)wave * TC;
   const uint32_t stride = (uint32_t)W * TC;
   const uint32_t skip = lo > t0 ? (lo - t0) / stride * stride : 0;
-  const uint32_t bs_mask = (1u << a.bs_log2) - 1u;
-  const uint32_t last_blk = (ctx - 1) >> a.bs_log2;
+  const uint32_t bs_mask = (1u << p_bs) - 1u;
+  const uint32_t last_blk = (ctx - 1) >> p_bs;
   const char *kbase =
       reinterpret_cast<const char *>(a.kc) + (size_t)kvh * a.head_stride * 4;
   const char *vbase =
@@ -1369,13 +1390,51 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
   const uint32_t newtok = (a.new_k != nullptr && ctx - 1 >= t0 && ctx - 1 < t1)
                               ? ctx - 1
                               : 0xFFFFFFFFu;
+  // The appended row and its slot are loaded ahead of the loop: a short
+  // context's whole time is a few round trips to memory.
+  const bool has_new = newtok != 0xFFFFFFFFu && wave == 0;
+  float4 nk[NL], nv[NL];
+  uint32_t new_blk = 0, new_off = 0;
+  if (has_new) {
+    new_blk = sload(a.new_blk + b);
+    new_off = sload(a.new_off + b);
+    const size_t src = ((size_t)b * a.n_kv + kvh) * HD;
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const uint32_t e0 = (j * R + c) * 4;
+      if (a.new_f32) {
+        nk[j] = *reinterpret_cast<const float4 *>(
+            static_cast<const float *>(a.new_k) + src + e0);
+        nv[j] = *reinterpret_cast<const float4 *>(
+            static_cast<const float *>(a.new_v) + src + e0);
+      } else {
+        const uint2 kh = *reinterpret_cast<const uint2 *>(
+            static_cast<const uint16_t *>(a.new_k) + src + e0);
+        const uint2 vh = *reinterpret_cast<const uint2 *>(
+            static_cast<const uint16_t *>(a.new_v) + src + e0);
+        const h2 k01 = as_h2(kh.x), k23 = as_h2(kh.y);
+        const h2 v01 = as_h2(vh.x), v23 = as_h2(vh.y);
+        nk[j] = make_float4((float)k01.x, (float)k01.y, (float)k23.x,
+                            (float)k23.y);
+        nv[j] = make_float4((float)v01.x, (float)v01.y, (float)v23.x,
+                            (float)v23.y);
+      }
+    }
+  }
+  // Block ids by scalar loads, a chunk ahead.
+  auto fetch_ids = [&](uint32_t ch) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      ids[u] = table[min((ch + u * RPL) >> p_bs, last_blk)];
+  };
+  if (skip || last_blk < ((first + TC - 1) >> p_bs)) fetch_ids(first + skip);
   for (uint32_t ch = first + skip; ch < t1; ch += stride) {
     float4 kr[U][NL], vr[U][NL];
     bool valid[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const uint32_t tb = ch + u * RPL;
-      const uint32_t id = table[min(tb >> a.bs_log2, last_blk)];
+      const uint32_t id = ids[u];
       const uint32_t tok = tb + rg;
       valid[u] = id < a.num_blocks && tok >= lo && tok < t1 && tok != newtok;
       const char *row = (uint64_t)(id < a.num_blocks ? id : 0u) * blk_bytes +
@@ -1392,6 +1451,7 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
                                __uint_as_float(vb.z), __uint_as_float(vb.w));
       }
     }
+    fetch_ids(ch + stride);
     // Keep the chunk's loads issued together ahead of the math (without
     // this fence the scheduler may pair each load with its first use).
     __builtin_amdgcn_sched_barrier(0);
@@ -1432,35 +1492,12 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
       }
     }
   }
-  if (newtok != 0xFFFFFFFFu && wave == 0) {
+  if (has_new) {
     // The appended row (f32 source copied, f16 widened exactly, as the
     // append does): stored by sub-group 0's row group 0, and one more key
     // of row group 0's softmax state.
-    float4 nk[NL], nv[NL];
-    const size_t src = ((size_t)b * a.n_kv + kvh) * HD;
-#pragma unroll
-    for (int j = 0; j < NL; ++j) {
-      const uint32_t e0 = (j * R + c) * 4;
-      if (a.new_f32) {
-        nk[j] = *reinterpret_cast<const float4 *>(
-            static_cast<const float *>(a.new_k) + src + e0);
-        nv[j] = *reinterpret_cast<const float4 *>(
-            static_cast<const float *>(a.new_v) + src + e0);
-      } else {
-        const uint2 kh = *reinterpret_cast<const uint2 *>(
-            static_cast<const uint16_t *>(a.new_k) + src + e0);
-        const uint2 vh = *reinterpret_cast<const uint2 *>(
-            static_cast<const uint16_t *>(a.new_v) + src + e0);
-        const h2 k01 = as_h2(kh.x), k23 = as_h2(kh.y);
-        const h2 v01 = as_h2(vh.x), v23 = as_h2(vh.y);
-        nk[j] = make_float4((float)k01.x, (float)k01.y, (float)k23.x,
-                            (float)k23.y);
-        nv[j] = make_float4((float)v01.x, (float)v01.y, (float)v23.x,
-                            (float)v23.y);
-      }
-    }
     if (sub == 0 && rg == 0) {
-      const uint32_t nb = a.new_blk[b], no = a.new_off[b];
+      const uint32_t nb = new_blk, no = new_off;
       if (nb < a.num_blocks && no < a.block_size) {
         const size_t dst = (size_t)nb * a.block_stride +
                            (size_t)kvh * a.head_stride + (size_t)no * HD;
@@ -1562,18 +1599,25 @@ __global__ void __launch_bounds__(256) decode_f32_kernel(DecodeArgs a) {
 }
 
 // Reduction pass (only for sequences split over several partitions): one
-// wave per (sequence, query head) merges its partitions: M = max m_i,
+// workgroup per (sequence, query head) merges its partitions: M = max m_i,
 // out = sum_i 2^(m_i - M) acc_i / sum_i 2^(m_i - M) l_i. Partitions that saw
-// no visible key carry l = 0 and are skipped.
+// no visible key carry l = 0 and are skipped. Bound by the launch and its
+// round trips to memory: a wave loads eight partitions' (m, l) and partials
+// at once, and with more than eight partitions four waves share them, merged
+// through LDS (25 partitions of Qwen3-0.6B heads:
+// 4.8 -> 4.0 us).
 template <int HD>
-__global__ void __launch_bounds__(64) decode_reduce_kernel(
+__global__ void __launch_bounds__(256) decode_reduce_kernel(
     const uint4 *p_reds, const float *p_ml, const float *p_acc,
     uint32_t p_nh, DecodeArgs a) {
   // (Leading arguments preloaded into SGPRs by the build; a holds the same
   // values.)
   constexpr int EPL = HD / 64 > 0 ? HD / 64 : 1;  // elements per lane
+  __shared__ float red_s[4][HD + 2];
   const uint32_t h = blockIdx.x;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t W = blockDim.x >> 6;
   uint32_t b, slot0, np;
   if (p_reds) {
     // The row is wave-uniform: scalar loads (constant address space).
@@ -1594,28 +1638,35 @@ __global__ void __launch_bounds__(64) decode_reduce_kernel(
   const float *accp = p_acc + ((size_t)slot0 * p_nh + h) * HD;
   const size_t acc_step = (size_t)p_nh * HD;
   const size_t hrow = (size_t)b * p_nh + h;
-  if (np <= 8) {
-    // Few partitions (the common case): every (m, l) pair (uniform loads)
-    // and every partial row are fetched at once, one round trip in all.
+  // This wave's partitions, eight at a time: one round trip.
+  const uint32_t per = (np + W - 1) / W;
+  const uint32_t p1 = min(np, (wave + 1) * per);
+  float acc[EPL], M = kNegBig, L = 0.f;
+#pragma unroll
+  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+  for (uint32_t c = wave * per; c < p1; c += 8) {
     float m[8], l[8], x[8][EPL];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const bool live = (uint32_t)k < np;
-      m[k] = live ? ml[k * ml_step] : kNegBig;
-      l[k] = live ? ml[k * ml_step + 1] : 0.f;
+      const bool live = c + k < p1;
+      const uint32_t p = c + k;
+      m[k] = live ? ml[p * ml_step] : kNegBig;
+      l[k] = live ? ml[p * ml_step + 1] : 0.f;
 #pragma unroll
       for (int e = 0; e < EPL; ++e) {
         const int d = lane * EPL + e;
-        x[k][e] = live && d < HD ? accp[k * acc_step + d] : 0.f;
+        x[k][e] = live && d < HD ? accp[p * acc_step + d] : 0.f;
       }
     }
-    float M = kNegBig;
+    float mx = M;
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (l[k] != 0.f) M = fmaxf(M, m[k]);
-    float acc[EPL], L = 0.f;
+      if (l[k] != 0.f) mx = fmaxf(mx, m[k]);
+    const float corr = __builtin_amdgcn_exp2f(M - mx);
+    M = mx;
+    L *= corr;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
+    for (int e = 0; e < EPL; ++e) acc[e] *= corr;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       // (l = 0: a partition that saw no visible key stays out)
@@ -1624,71 +1675,31 @@ __global__ void __launch_bounds__(64) decode_reduce_kernel(
 #pragma unroll
       for (int e = 0; e < EPL; ++e) acc[e] += w != 0.f ? w * x[k][e] : 0.f;
     }
-    const float inv = L > 0.f ? 1.0f / L : 0.f;
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) {
-      const int d = lane * EPL + e;
-      if ((uint32_t)d < a.hd) a.out[hrow * a.hd + d] = acc[e] * inv;
-    }
-    return;
   }
-  // Lane i holds partition c + i's (m, l) for the 64-partition chunk at c;
-  // M comes first, then every partial is weighted by 2^(m_i - M): the loads
-  // of different partitions are independent, so they are all in flight at
-  // once instead of one round trip per partition.
-  float M = kNegBig;
-  for (uint32_t c = 0; c < np; c += 64) {
-    const uint32_t p = c + lane;
-    if (p < np && ml[p * ml_step + 1] != 0.f) M = fmaxf(M, ml[p * ml_step]);
-  }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) M = fmaxf(M, __shfl_xor(M, o));
-  float acc[EPL];
-#pragma unroll
-  for (int e = 0; e < EPL; ++e) acc[e] = 0.f;
-  float L = 0.f;
-  for (uint32_t c = 0; c < np; c += 64) {
-    const uint32_t p = c + lane;
-    float w = 0.f;
-    if (p < np) {
-      const float lp = ml[p * ml_step + 1];
-      // (l = 0: a partition that saw no visible key)
-      if (lp != 0.f) w = __builtin_amdgcn_exp2f(ml[p * ml_step] - M);
-      L += lp * w;
-    }
-    const uint32_t n = min(np - c, 64u);
-    // Eight partitions per pass: their loads all issue before any is used.
-    auto add = [&](uint32_t i, const float (&x)[EPL]) {
-      const float wi =
-          __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), i));
+  if (W > 1) {
+    if (wave > 0) {
+      if (lane == 0) {
+        red_s[wave][HD] = M;
+        red_s[wave][HD + 1] = L;
+      }
 #pragma unroll
       for (int e = 0; e < EPL; ++e)
-        acc[e] += wi != 0.f ? wi * x[e] : 0.f;  // skipped partials stay out
-    };
-    auto fetch = [&](uint32_t i, float (&x)[EPL]) {
-      const float *src = accp + (size_t)(c + i) * acc_step;
-#pragma unroll
-      for (int e = 0; e < EPL; ++e) {
-        const int d = lane * EPL + e;
-        x[e] = d < HD ? src[d] : 0.f;
-      }
-    };
-    uint32_t i = 0;
-    for (; i + 8 <= n; i += 8) {
-      float x[8][EPL];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) fetch(i + k, x[k]);
-#pragma unroll
-      for (int k = 0; k < 8; ++k) add(i + k, x[k]);
+        if (lane * EPL + e < HD) red_s[wave][lane * EPL + e] = acc[e];
     }
-    for (; i < n; ++i) {
-      float x[EPL];
-      fetch(i, x);
-      add(i, x);
+    __syncthreads();
+    if (wave > 0) return;
+    for (uint32_t w = 1; w < W; ++w) {
+      const float mw = red_s[w][HD], mx = fmaxf(M, mw);
+      const float ca = __builtin_amdgcn_exp2f(M - mx);
+      const float cb = __builtin_amdgcn_exp2f(mw - mx);
+      M = mx;
+      L = L * ca + red_s[w][HD + 1] * cb;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e)
+        if (lane * EPL + e < HD)
+          acc[e] = acc[e] * ca + red_s[w][lane * EPL + e] * cb;
     }
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) L += __shfl_xor(L, o);
   const float inv = L > 0.f ? 1.0f / L : 0.f;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
@@ -1733,9 +1744,6 @@ void subgroups(uint32_t group, uint32_t *n_sub, uint32_t *gt) {
   *gt = div_up(group, *n_sub);
 }
 
-// Tokens per context partition: the smallest power of two >= 256 for which
-// the grid has at most ~8192 partition waves (32 per CU on 256 CUs), so long
-// contexts keep enough waves in flight without a large reduction.
 // Tuning overrides (RVKV_DECODE_PART_TOKENS, RVKV_DECODE_UNROLL); 0 = auto.
 uint32_t env_u32(const char *name) {
   const char *v = getenv(name);
@@ -1779,14 +1787,42 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
   uint32_t n_sub, gt;
   subgroups(group ? group : 1, &n_sub, &gt);
   const uint64_t pairs = (uint64_t)batch * p->n_kv * n_sub;
-  // Enough workgroups for two per CU (256 CUs); a whole context per
-  // workgroup whenever the batch alone provides that many.
+  // Two workgroups a CU, in whole 64-token steps (2 x 12345 tokens of
+  // Qwen3-0.6B heads: 448 partitions' workgroups 20.9 us, the next power of
+  // two's 400 21.4 us; 8 x 5000, f32 cells: 512 against 320, 53.3 against
+  // 57.8 us; for 768 or 1024 workgroups the same or slower). At least 256
+  // tokens, or 128 where a key is 1 KiB (3 x 600 tokens of gemma-3 heads:
+  // 17.2 -> 11.1 us). Large groups at head_dim 256 keep powers of two and no
+  // other rule: rvkv_paged_decode_noalloc refuses them by their partials'
+  // size, which stays what it is.
   const uint64_t want = 512;
   const uint64_t parts = pairs >= want ? 1 : (want + pairs - 1) / pairs;
   const uint64_t per = (max_ctx + parts - 1) / parts;
-  uint32_t P = 256;
-  while (P < per && P < (1u << 30)) P <<= 1;
-  return P;
+  const bool big = p->head_dim > 128;
+  uint64_t P = big && gt <= 4 ? 128 : 256;
+  if (big && gt > 4) {
+    while (P < per && P < (1u << 30)) P <<= 1;
+    return (uint32_t)P;
+  }
+  P = std::max<uint64_t>(P, (per + 63) / 64 * 64);
+  // One workgroup a sequence and KV head saves the reduction launch, ~5 us.
+  // A workgroup streams ~60 KB/us (~40 with four waves), the chip 5.3 MB/us,
+  // of which a ragged batch asks perhaps 40 % (max_ctx is its longest): one
+  // when that costs less than cutting and 5 us. (us a layer, cut with the
+  // reduction and its launch gap against one: SmolLM2 heads f32, 8 x 512,
+  // 14.3 / 9.6; Qwen3-0.6B heads 1 x 500 13.9 / 10.3, 1 x 1000 12.3 / 14.7,
+  // 20 x 1500 31.0 / 25.9, 40 x 4500 170 / 141; gemma-3 heads f32, 100
+  // ragged to 1500, 42 / 59.)
+  const double row = 2.0 * p->head_dim * p->elem_bytes;
+  const int hdp = (int)decode_hd(p->head_dim);
+  const double rate =
+      decode_max_waves(hdp, (int)gt, p->f32()) > 4 ? 60e3 : 40e3;
+  const double all = row * max_ctx * pairs * 0.4 / 5.3e6;
+  const double one = std::max(row * max_ctx / rate, all);
+  const double cut =
+      std::max(row * (double)std::min<uint64_t>(P, max_ctx) / rate, all) + 5.0;
+  if (one <= cut) P = std::max<uint64_t>(P, ((uint64_t)max_ctx + 63) / 64 * 64);
+  return (uint32_t)P;
 }
 
 // Short items: even the longest workgroup has under 192 context tokens.
@@ -1871,13 +1907,25 @@ void launch_decode(const DecodeArgs &a, dim3 grid, hipStream_t st) {
   // plan's ragged items keep four: churn's long-item phase was no faster.)
   if (!forced_w && !a.items && u8 && W == 4 && wgs > 512 && wgs <= 1024)
     W = 2;
+  // More waves where the workgroups alone leave the chip idle, until each has
+  // one chunk or ~2048 are resident (SmolLM2 heads f32, 80 workgroups of 256
+  // tokens: 9.6 -> 8.0 us; 400 workgroups of 512 with eight waves each, past
+  // that: 21.4 -> 23.7 us).
+  if (!forced_w && W == 4) {
+    const uint32_t tc = (a.f32cache ? 4u * 64u / (HD / (HD >= 256 ? 8 : 4))
+                                    : (u8 ? 8u : u2 ? 2u : 4u) * 64u / (HD / 8));
+    while (W < (uint32_t)decode_max_waves(HD, GT, a.f32cache) &&
+           W * tc < a.max_tokens && wgs * W <= 1024)
+      W *= 2;
+  }
   // (m, l) pairs rounded up to 16 bytes, then the accumulator rows; at
   // least the f32 kernel's W * GT * (HD + 2) floats.
   const size_t lds =
       (((size_t)W * GT * 2 + 3) / 4 * 4 + (size_t)W * GT * HD) * sizeof(float);
   if (a.f32cache)
     hipLaunchKernelGGL((decode_f32_kernel<HD, GT>), grid, dim3(64 * W), lds, st,
-                       a);
+                       a.items, a.tables, a.ctx_lens, a.max_blocks, a.bs_log2,
+                       a.part_tokens, a);
   else if (a.hd != HD)  // a head_dim below HD: rows read element by element
     hipLaunchKernelGGL((decode_part_kernel<HD, GT, 4, 1, true>), grid,
                        dim3(64 * W), lds, st, a.items, a.tables,
@@ -2274,6 +2322,20 @@ int check_ws(const char *op, void *ws, size_t ws_bytes, size_t need) {
   return RVKV_OK;
 }
 
+// The reduction of split sequences: rgrid = (query heads, split sequences).
+int launch_reduce(const char *op, const DecodeArgs &a, uint32_t hd,
+                  dim3 rgrid, hipStream_t st) {
+  const dim3 block(a.max_parts > 8 ? 256 : 64);
+  switch (hd) {
+    case 32: hipLaunchKernelGGL(decode_reduce_kernel<32>, rgrid, block, 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
+    case 64: hipLaunchKernelGGL(decode_reduce_kernel<64>, rgrid, block, 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
+    case 128: hipLaunchKernelGGL(decode_reduce_kernel<128>, rgrid, block, 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
+    default: hipLaunchKernelGGL(decode_reduce_kernel<256>, rgrid, block, 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
+  }
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess ? RVKV_OK : hip_fail(op, e);
+}
+
 // Launches the partition kernel on `grid` and, when some sequence is split,
 // the reduction kernel on `rgrid`.
 int launch_decode_pair(const char *op, const DecodeArgs &a, uint32_t hd,
@@ -2285,26 +2347,7 @@ int launch_decode_pair(const char *op, const DecodeArgs &a, uint32_t hd,
     case 128: dispatch_gt<128>(gt, a, grid, st); break;
     default: dispatch_gt<256>(gt, a, grid, st); break;
   }
-  if (reduce) {
-    switch (hd) {
-      case 32: hipLaunchKernelGGL(decode_reduce_kernel<32>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-      case 64: hipLaunchKernelGGL(decode_reduce_kernel<64>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-      case 128: hipLaunchKernelGGL(decode_reduce_kernel<128>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-      default: hipLaunchKernelGGL(decode_reduce_kernel<256>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-    }
-  }
-  hipError_t e = hipGetLastError();
-  return e == hipSuccess ? RVKV_OK : hip_fail(op, e);
-}
-
-int launch_reduce(const char *op, const DecodeArgs &a, uint32_t hd,
-                  dim3 rgrid, hipStream_t st) {
-  switch (hd) {
-    case 32: hipLaunchKernelGGL(decode_reduce_kernel<32>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-    case 64: hipLaunchKernelGGL(decode_reduce_kernel<64>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-    case 128: hipLaunchKernelGGL(decode_reduce_kernel<128>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-    default: hipLaunchKernelGGL(decode_reduce_kernel<256>, rgrid, dim3(64), 0, st, a.reds, a.ws_ml, a.ws_acc, a.n_heads, a); break;
-  }
+  if (reduce) return launch_reduce(op, a, hd, rgrid, st);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? RVKV_OK : hip_fail(op, e);
 }
@@ -2324,7 +2367,7 @@ struct rvkv_decode_plan {
   uint32_t batch, n_heads, n_kv, head_dim, max_ctx;
   int32_t window;
   uint32_t part_tokens, n_items, n_reds, n_slots, avg_tokens = 0,
-      max_tokens = 0;
+      max_tokens = 0, max_parts = 0;
   uint4 *d_buf = nullptr;   // items, reduction rows, group lists (device)
   // Pinned staging copies of the same, used in turn: an update waits only
   // for the upload kNStage updates back, so the host can build a few steps
@@ -2701,6 +2744,8 @@ int plan_build(rvkv_decode_plan *pl, const uint32_t *ctx_lens_host,
   pl->max_tokens = 0;
   for (const uint4 &it : items)
     pl->max_tokens = std::max(pl->max_tokens, it.z > it.y ? it.z - it.y : 0u);
+  pl->max_parts = 0;
+  for (const uint4 &r : reds) pl->max_parts = std::max(pl->max_parts, r.z);
   pl->n_items = (uint32_t)items.size();
   pl->n_reds = (uint32_t)reds.size();
   pl->n_slots = slots;
@@ -2895,6 +2940,7 @@ int paged_decode_ws(const char *op, const rvkv_pool *pool, uint32_t layer,
   a.ws_ml = w.n_parts > 1 ? (float *)((char *)ws + w.ml_off) : nullptr;
   a.part_tokens = partition_tokens(pool, batch, n_heads, max_ctx_len);
   a.n_parts = w.n_parts;
+  a.max_parts = w.n_parts;
   a.avg_tokens = a.part_tokens < max_ctx_len ? a.part_tokens : max_ctx_len;
   a.max_tokens = a.avg_tokens;
   const dim3 grid(w.n_parts, pool->n_kv * a.n_sub, batch);
@@ -3007,6 +3053,7 @@ int rvkv_paged_decode_planned(const rvkv_pool *pool,
   a.part_tokens = plan->part_tokens;
   a.avg_tokens = plan->avg_tokens;
   a.max_tokens = plan->max_tokens;
+  a.max_parts = plan->max_parts;
   a.n_parts = 1;
   if (rvkv_detail::mfma_decode_wanted(pool, plan->n_heads))
     return planned_mfma(op, pool, plan, layer, a, max_blocks, scale);
@@ -3077,6 +3124,7 @@ int rvkv_decode_step(rvkv_pool *pool, const rvkv_decode_plan *plan,
     a.part_tokens = plan->part_tokens;
     a.avg_tokens = plan->avg_tokens;
     a.max_tokens = plan->max_tokens;
+    a.max_parts = plan->max_parts;
     a.n_parts = 1;
     if (rvkv_detail::mfma_decode_wanted(pool, n_heads))
       return planned_mfma(op, pool, plan, layer, a, max_blocks, scale);
@@ -3094,6 +3142,7 @@ int rvkv_decode_step(rvkv_pool *pool, const rvkv_decode_plan *plan,
   a.ws_ml = w.n_parts > 1 ? (float *)((char *)ws + w.ml_off) : nullptr;
   a.part_tokens = partition_tokens(pool, batch, n_heads, max_ctx_len);
   a.n_parts = w.n_parts;
+  a.max_parts = w.n_parts;
   a.avg_tokens = a.part_tokens < max_ctx_len ? a.part_tokens : max_ctx_len;
   a.max_tokens = a.avg_tokens;
   if (rvkv_detail::mfma_decode_wanted(pool, n_heads))

@@ -1702,6 +1702,49 @@ def test_prefill_large_scores(hd):
     assert np.isfinite(out).all() and np.abs(out - want).max() < ATOL
 
 
+@pytest.mark.parametrize("hd,G,batch,ctx,dtype", [
+    (64, 3, 8, 512, torch.float32),     # one partition of 16 waves
+    (64, 2, 1, 33, torch.float16),      # fewer chunks than waves
+    (128, 2, 1, 500, torch.float16),    # one partition of eight waves
+    (128, 2, 1, 1025, torch.float16),   # partitions of 256, one token over
+    (128, 7, 2, 700, torch.float32),
+    (128, 2, 2, 12345, torch.float16),  # partitions not a power of two
+    (128, 1, 3, 9000, torch.float32),   # reduction of > 32 partitions
+    (256, 4, 3, 600, torch.float16),    # partitions of 128
+    (256, 4, 5, 1100, torch.float32),
+    (256, 8, 3, 3000, torch.float16),   # four waves, powers of two
+])
+def test_decode_partition_rule(hd, G, batch, ctx, dtype):
+    """Unplanned decode over every kind of partition and workgroup width,
+    plain and with the fused append, against float64 over the raw cache."""
+    nkv, bs = 2, 16
+    rng = np.random.default_rng(ctx + hd)
+    lens = rng.integers(1, ctx + 1, batch)
+    lens[0] = ctx
+    mb = -(-ctx // bs)
+    st = HipKvStorage(1, batch * mb, bs, nkv, hd, dtype=dtype)
+    at = torch.arange(batch * mb * bs, device="cuda")
+    rnd = lambda *s: torch.randn(*s, device="cuda").to(dtype)
+    st.write_tokens(0, (at // bs).int(), (at % bs).int(),
+                    rnd(len(at), nkv, hd), rnd(len(at), nkv, hd))
+    tables = rng.permutation(batch * mb).reshape(batch, mb).astype(np.uint32)
+    t, n = dev_u32(tables), dev_u32(lens)
+    q = torch.randn(batch, nkv * G, hd, device="cuda")
+    tol = 2e-5 if dtype == torch.float32 else ATOL
+    for window in (0, 200):
+        out = st.paged_decode(0, q, t, n, ctx, window=window)
+        want = _prefill_f64(st, q[:, None], tables, lens - 1, lens, window)
+        assert (out - want[:, 0]).abs().max() < tol, window
+        assert torch.equal(st.paged_decode(0, q, t, n, ctx, window=window),
+                           out)
+    k, v = (torch.randn(batch, nkv, hd, device="cuda") for _ in range(2))
+    pos = lens - 1
+    out = st.decode_step(0, k, v, dev_u32(tables[range(batch), pos // bs]),
+                         dev_u32(pos % bs), q, t, n, ctx)
+    want = _prefill_f64(st, q[:, None], tables, lens - 1, lens, 0)
+    assert (out - want[:, 0]).abs().max() < tol
+
+
 def _prefill_f64(st, q, tables, prior, read, window):
     """Prefill attention in float64 from the raw cache (keys behind an
     out-of-range id hidden), on the GPU."""

@@ -2179,3 +2179,21 @@ def test_graph_capture_prep_prefill_argmax():
         for w in (0, 1):
             assert torch.equal(pools[0].read_blocks(0, w, ids),
                                pools[1].read_blocks(0, w, ids)), (rep, w)
+
+
+def test_backend_rope_table_grows():
+    """A forward past the RoPE table's end (a decode row beside it) gives the
+    bits of a backend whose table held those positions from the start."""
+    from rvllm_amd.attn_model import AttnModelConfig, HipBackend, init_weights
+    from rvllm_amd.engine import BatchItem
+    out = []
+    for context in (64, 4096):
+        cfg = AttnModelConfig(context_length=context)
+        be = HipBackend(cfg, init_weights(cfg), 40, 16)
+        for l in range(cfg.n_layers):
+            fill_layer(be.st, l, seed=l)
+        items = [BatchItem(0, [5], [(3, 2)], [1, 2, 3], 35, 34),
+                 BatchItem(1, [9], [(20, 1)], list(range(12, 21)), 130, 129)]
+        be.forward_sample(items, False, [None] * 2)
+        out.append(be.last_logits.clone())
+    assert torch.equal(*out)

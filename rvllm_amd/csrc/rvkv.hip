@@ -1750,6 +1750,33 @@ uint32_t env_u32(const char *name) {
   return v ? (uint32_t)strtoul(v, nullptr, 10) : 0u;
 }
 
+// KB/us that one decode workgroup streams where the chip is idle: eight and
+// more waves, four, or four on the matrix cores (a wave's 32-key tiles follow
+// each other).
+double decode_rate(const rvkv_pool *p, uint32_t n_heads, uint32_t gt) {
+  if (rvkv_detail::mfma_decode_wanted(p, n_heads)) return 29e3;
+  return decode_max_waves((int)decode_hd(p->head_dim), (int)gt, p->f32()) > 4
+             ? 60e3
+             : 40e3;
+}
+
+// Whether a decode of sequences of up to `longest` tokens, `all` (sequence,
+// KV head) tokens in all, runs faster as one workgroup a sequence and KV head
+// than in partitions of `part` tokens: cutting costs the reduction launch,
+// ~5 us; the chip streams 5.3 MB/us. (us a layer, cut with the reduction and
+// its launch gap against one: SmolLM2 heads f32, 8 x 512, 14.3 / 9.6;
+// Qwen3-0.6B heads 1 x 500 13.9 / 10.3, 1 x 1000 12.3 / 14.7, 20 x 1500
+// 31.0 / 25.9, 40 x 4500 170 / 141; gemma-3 heads f32, 100 ragged to 1500,
+// 42 / 59. Matrix cores, Llama-3.2-1B heads: 4 x 400 11.3 / 8.6, 4 x 760 13.1
+// / 11.8, 40 x 630 25.5 / 16.5, 1 x 1000 12.3 / 13.)
+bool one_workgroup(const rvkv_pool *p, double rate, double longest,
+                   double part, double all) {
+  const double row = 2.0 * p->head_dim * p->elem_bytes;  // bytes a token
+  const double shared = row * all / 5.3e6;
+  return std::max(row * longest / rate, shared) <=
+         std::max(row * std::min(part, longest) / rate, shared) + 5.0;
+}
+
 // The matrix-core decode without a plan: waves a partition (its keys split
 // over them, merged in the workgroup) and partition size. Four waves a
 // partition below 2048 (sequence, KV head) pairs (as for plan items), then
@@ -1761,7 +1788,8 @@ uint32_t env_u32(const char *name) {
 // wave a sequence, 326 us.) RVKV_DECODE_KSPLIT=1|2|4 overrides; it is read
 // at every call, so a test can take each width (each call sizes and checks
 // its workspace against the same reading).
-uint32_t mfma_uniform_parts(uint64_t pairs, uint32_t max_ctx,
+uint32_t mfma_uniform_parts(const rvkv_pool *p, uint32_t n_heads,
+                            uint64_t pairs, uint32_t max_ctx,
                             uint32_t *ksplit) {
   const uint32_t forced_k = env_u32("RVKV_DECODE_KSPLIT");
   *ksplit = forced_k == 1 || forced_k == 2 || forced_k == 4
@@ -1772,6 +1800,10 @@ uint32_t mfma_uniform_parts(uint64_t pairs, uint32_t max_ctx,
   const uint64_t per = (max_ctx + parts - 1) / parts;
   uint32_t P = 256;
   while (P < per && P < 4096) P <<= 1;
+  if (*ksplit == 4 && max_ctx <= 4096 &&
+      one_workgroup(p, decode_rate(p, n_heads, 1), max_ctx, P,
+                    0.4 * max_ctx * pairs))
+    P = std::max(P, (max_ctx + 255) / 256 * 256);
   return P;
 }
 
@@ -1781,7 +1813,8 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
   if (forced >= 256 && forced % 256 == 0) return forced;
   if (rvkv_detail::mfma_decode_wanted(p, n_heads)) {
     uint32_t ksplit;
-    return mfma_uniform_parts((uint64_t)batch * p->n_kv, max_ctx, &ksplit);
+    return mfma_uniform_parts(p, n_heads, (uint64_t)batch * p->n_kv, max_ctx,
+                              &ksplit);
   }
   uint32_t group = n_heads / (p->n_kv ? p->n_kv : 1);
   uint32_t n_sub, gt;
@@ -1805,23 +1838,10 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
     return (uint32_t)P;
   }
   P = std::max<uint64_t>(P, (per + 63) / 64 * 64);
-  // One workgroup a sequence and KV head saves the reduction launch, ~5 us.
-  // A workgroup streams ~60 KB/us (~40 with four waves), the chip 5.3 MB/us,
-  // of which a ragged batch asks perhaps 40 % (max_ctx is its longest): one
-  // when that costs less than cutting and 5 us. (us a layer, cut with the
-  // reduction and its launch gap against one: SmolLM2 heads f32, 8 x 512,
-  // 14.3 / 9.6; Qwen3-0.6B heads 1 x 500 13.9 / 10.3, 1 x 1000 12.3 / 14.7,
-  // 20 x 1500 31.0 / 25.9, 40 x 4500 170 / 141; gemma-3 heads f32, 100
-  // ragged to 1500, 42 / 59.)
-  const double row = 2.0 * p->head_dim * p->elem_bytes;
-  const int hdp = (int)decode_hd(p->head_dim);
-  const double rate =
-      decode_max_waves(hdp, (int)gt, p->f32()) > 4 ? 60e3 : 40e3;
-  const double all = row * max_ctx * pairs * 0.4 / 5.3e6;
-  const double one = std::max(row * max_ctx / rate, all);
-  const double cut =
-      std::max(row * (double)std::min<uint64_t>(P, max_ctx) / rate, all) + 5.0;
-  if (one <= cut) P = std::max<uint64_t>(P, ((uint64_t)max_ctx + 63) / 64 * 64);
+  // (a ragged batch holds perhaps 40 % of what its longest sequence says)
+  if (one_workgroup(p, decode_rate(p, n_heads, gt), max_ctx, P,
+                    0.4 * max_ctx * pairs))
+    P = std::max<uint64_t>(P, ((uint64_t)max_ctx + 63) / 64 * 64);
   return (uint32_t)P;
 }
 
@@ -2429,11 +2449,12 @@ int plan_build(rvkv_decode_plan *pl, const uint32_t *ctx_lens_host,
   const int32_t window = pl->window;
   // Visible tokens per sequence: [lo_b, ctx_b), lo_b from the window.
   uint64_t total = 0;
-  uint32_t max_ctx = 1;
+  uint32_t max_ctx = 1, longest = 0;
   for (uint32_t b = 0; b < batch; ++b) {
     const uint32_t n = ctx_lens_host[b];
     const uint32_t lo = (window > 0 && n > (uint32_t)window) ? n - window : 0;
     total += n - lo;
+    longest = std::max(longest, n - lo);
     if (n > max_ctx) max_ctx = n;
   }
   // Tokens per work item: about one sequence, but at least enough that the
@@ -2474,10 +2495,17 @@ int plan_build(rvkv_decode_plan *pl, const uint32_t *ctx_lens_host,
   // first (longest first) finishes in the launch's tail, when the bandwidth
   // is its own; the few long survivors of a churning batch are still cut
   // into items near the typical length.
-  const uint32_t whole_max =
+  uint32_t whole_max =
       mfma ? 0u
            : (uint32_t)std::min(std::min(4.0 * (double)total / batch, hi_p),
                                 2.0 * P);
+  // A launch that leaves workgroup slots idle: no sequence is cut where the
+  // reduction would cost more (Qwen3-0.6B heads, 30 ragged to 1500: 24.3 ->
+  // 22.1 us; Llama-3.2-1B heads, 8 ragged to 500: 14 -> 9.4 us).
+  if (batch * n_hy <= 512 &&
+      one_workgroup(pool, decode_rate(pool, pl->n_heads, gt), longest, P,
+                    (double)total * n_hy))
+    whole_max = longest;
   auto split = [&](uint32_t start, uint32_t n, uint32_t *step_out) {
     const uint32_t span = n - start;
     if (span <= whole_max) {
@@ -2867,7 +2895,8 @@ int uniform_mfma(const char *op, const rvkv_pool *pool, uint32_t layer,
   uint32_t ksplit = 1;
   static const uint32_t forced = env_u32("RVKV_DECODE_PART_TOKENS");
   if (!forced)
-    mfma_uniform_parts((uint64_t)batch * pool->n_kv, a.ctx_cap, &ksplit);
+    mfma_uniform_parts(pool, a.n_heads, (uint64_t)batch * pool->n_kv, a.ctx_cap,
+                       &ksplit);
   int rc = rvkv_detail::mfma_decode(
       pool, layer, a.q, a.tables, a.ctx_lens, a.max_blocks, a.n_heads, scale,
       a.window, nullptr, batch * a.n_parts, a.ws_acc, a.ws_ml, a.out,

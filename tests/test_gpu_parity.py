@@ -1713,6 +1713,8 @@ def test_prefill_large_scores(hd):
     (256, 4, 3, 600, torch.float16),    # partitions of 128
     (256, 4, 5, 1100, torch.float32),
     (256, 8, 3, 3000, torch.float16),   # four waves, powers of two
+    (64, 4, 4, 760, torch.float16),     # matrix cores, one item a sequence
+    (64, 7, 1, 1000, torch.float16),    # matrix cores, partitions
 ])
 def test_decode_partition_rule(hd, G, batch, ctx, dtype):
     """Unplanned decode over every kind of partition and workgroup width,
@@ -1743,6 +1745,11 @@ def test_decode_partition_rule(hd, G, batch, ctx, dtype):
                          dev_u32(pos % bs), q, t, n, ctx)
     want = _prefill_f64(st, q[:, None], tables, lens - 1, lens, 0)
     assert (out - want[:, 0]).abs().max() < tol
+    for window in (0, 200):  # the same through a plan
+        plan = HipDecodePlan(st, lens, nkv * G, window=window)
+        want = _prefill_f64(st, q[:, None], tables, lens - 1, lens, window)
+        out = st.paged_decode_planned(0, plan, q, t, n)
+        assert (out - want[:, 0]).abs().max() < tol
 
 
 def _prefill_f64(st, q, tables, prior, read, window):

@@ -2204,3 +2204,20 @@ def test_backend_rope_table_grows():
         be.forward_sample(items, False, [None] * 2)
         out.append(be.last_logits.clone())
     assert torch.equal(*out)
+
+
+@pytest.mark.parametrize("rows,V", [(1, 4096), (1, 16388), (511, 4100),
+                                    (512, 4100), (700, 1003), (2, 4101)])
+def test_argmax_thread_counts(rows, V):
+    """Both workgroup sizes, aligned and odd rows, with ties in different
+    threads, waves and load groups: the lowest index wins."""
+    import ctypes
+    from rvllm_amd import _lib
+    x = torch.randn(rows, V, device="cuda").clamp_(max=1.0)  # many ties at 1
+    x[::3, V - 1] = 2.0
+    out = torch.empty(rows, dtype=torch.int32, device="cuda")
+    _lib.check(_lib.load().rvkv_argmax(
+        ctypes.c_void_p(x.data_ptr()), rows, V,
+        ctypes.c_void_p(out.data_ptr()),
+        ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)))
+    assert out.tolist() == orc.argmax_rows(x.cpu().numpy()).tolist()

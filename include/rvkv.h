@@ -281,8 +281,8 @@ int rvkv_decode_step(rvkv_pool *pool, const rvkv_decode_plan *plan,
  * The rotated q goes to q_out [rows, n_heads, hd] f32; k and v are rounded
  * to f16 (nearest-even; stored as they are in an f32 pool) and written to
  * (slot_block[i], slot_off[i]) of `layer`, as rvkv_append would. head_dim
- * even and <= 1024 (32, 64, 128 and 256 on the tuned kernel, others and f32
- * pools on a generic one); every float buffer 16-byte aligned (RVKV_EINVAL
+ * even and <= 1024 (32, 64, 128 and 256 on the tuned kernel, others on a
+ * generic one); every float buffer 16-byte aligned (RVKV_EINVAL
  * otherwise). Rows whose slot is
  * out of range still produce q_out but write no k/v. */
 int rvkv_attn_prep(rvkv_pool *pool, uint32_t layer, const float *q_in,

@@ -334,7 +334,8 @@ __device__ __forceinline__ uint32_t h2bits(float lo, float hi) {
   return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) |
          ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
 }
-__device__ __forceinline__ void st8h(uint16_t *p, const float *x) {
+__device__ __forceinline__ void st8c(float *p, const float *x) { st8(p, x); }
+__device__ __forceinline__ void st8c(_Float16 *p, const float *x) {
   *reinterpret_cast<uint4 *>(p) = make_uint4(
       h2bits(x[0], x[1]), h2bits(x[2], x[3]), h2bits(x[4], x[5]),
       h2bits(x[6], x[7]));
@@ -346,7 +347,9 @@ __device__ __forceinline__ void st8h(uint16_t *p, const float *x) {
 // T = HD/16 lanes of an item reduce the RMS sum of squares by xor shuffles.
 // Element arithmetic is the reference's, unfused (contract off): bias add,
 // x / rms * w, then x0*c - x1*s and x0*s + x1*c.
-template <int HD>
+// Cell: the cache's (f16 rounds k and v to nearest even, f32 stores them: on
+// an f32 pool 25 heads x 700 rows 6.9 us on the generic kernel, 4.4 here).
+template <int HD, typename Cell>
 __global__ void __launch_bounds__(256) attn_prep_kernel(PrepArgs a) {
 #pragma clang fp contract(off)
   constexpr int HALF = HD / 2;
@@ -382,10 +385,12 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(PrepArgs a) {
   const uint32_t blk = a.slot_block[row], off = a.slot_off[row];
   const bool slot_ok = blk < a.num_blocks && off < a.bs;
   const size_t dst = (((size_t)blk * a.n_kv + hh) * a.bs + off) * HD;
+  Cell *kc = reinterpret_cast<Cell *>(a.kc);
+  Cell *vc = reinterpret_cast<Cell *>(a.vc);
   if (is_v) {
     if (slot_ok) {
-      st8h(a.vc + dst + j, x0);
-      st8h(a.vc + dst + j + HALF, x1);
+      st8c(vc + dst + j, x0);
+      st8c(vc + dst + j + HALF, x1);
     }
     return;
   }
@@ -420,13 +425,13 @@ __global__ void __launch_bounds__(256) attn_prep_kernel(PrepArgs a) {
     st8(o + j, r0);
     st8(o + j + HALF, r1);
   } else if (slot_ok) {
-    st8h(a.kc + dst + j, r0);
-    st8h(a.kc + dst + j + HALF, r1);
+    st8c(kc + dst + j, r0);
+    st8c(kc + dst + j + HALF, r1);
   }
 }
 
 // attn_prep for the shapes attn_prep_kernel does not take (an even head_dim
-// other than 32/64/128/256, or f32 cells): one wave per (row, head slot),
+// other than 32/64/128/256): one wave per (row, head slot),
 // lane i owning the rotate-half pairs (p, p + hd/2) for p = i, i + 64, ...;
 // the same element arithmetic, the RMS sum reduced over the wave.
 template <typename Cell>
@@ -3185,6 +3190,17 @@ int rvkv_decode_step(rvkv_pool *pool, const rvkv_decode_plan *plan,
 
 namespace {
 
+template <typename Cell>
+void launch_prep(const PrepArgs &a, dim3 grid, uint32_t hd, hipStream_t st) {
+  const dim3 block(256);
+  switch (hd) {
+    case 32: hipLaunchKernelGGL((attn_prep_kernel<32, Cell>), grid, block, 0, st, a); break;
+    case 64: hipLaunchKernelGGL((attn_prep_kernel<64, Cell>), grid, block, 0, st, a); break;
+    case 128: hipLaunchKernelGGL((attn_prep_kernel<128, Cell>), grid, block, 0, st, a); break;
+    default: hipLaunchKernelGGL((attn_prep_kernel<256, Cell>), grid, block, 0, st, a); break;
+  }
+}
+
 // Shared by the split (q, k, v) and the fused (qkv) entry points; q and
 // k/v rows are q_stride / kv_stride floats apart.
 int attn_prep_impl(rvkv_pool *pool, uint32_t layer, const float *q_in,
@@ -3233,9 +3249,10 @@ int attn_prep_impl(rvkv_pool *pool, uint32_t layer, const float *q_in,
   const uint64_t items = (uint64_t)rows * (n_heads + 2 * pool->n_kv);
   if (items > 0xffffffffull)
     return fail(RVKV_EUNSUPPORTED, op, "too many rows for one launch");
-  if (pool->f32() || !hd_supported(hd)) {
-    if (items > 0x7fffffffull)
-      return fail(RVKV_EUNSUPPORTED, op, "too many rows for one launch");
+  // (the bound of the generic kernel, which f32 pools used to run)
+  if ((pool->f32() || !hd_supported(hd)) && items > 0x7fffffffull)
+    return fail(RVKV_EUNSUPPORTED, op, "too many rows for one launch");
+  if (!hd_supported(hd)) {
     const dim3 grid((uint32_t)items);
     if (pool->f32())
       hipLaunchKernelGGL(attn_prep_generic_kernel<float>, grid, dim3(64), 0,
@@ -3248,12 +3265,10 @@ int attn_prep_impl(rvkv_pool *pool, uint32_t layer, const float *q_in,
   }
   const uint32_t per_block = 256 / (hd / 16);
   const dim3 grid((uint32_t)((items + per_block - 1) / per_block));
-  switch (hd) {
-    case 32: hipLaunchKernelGGL(attn_prep_kernel<32>, grid, dim3(256), 0, pool->stream, a); break;
-    case 64: hipLaunchKernelGGL(attn_prep_kernel<64>, grid, dim3(256), 0, pool->stream, a); break;
-    case 128: hipLaunchKernelGGL(attn_prep_kernel<128>, grid, dim3(256), 0, pool->stream, a); break;
-    default: hipLaunchKernelGGL(attn_prep_kernel<256>, grid, dim3(256), 0, pool->stream, a); break;
-  }
+  if (pool->f32())
+    launch_prep<float>(a, grid, hd, pool->stream);
+  else
+    launch_prep<_Float16>(a, grid, hd, pool->stream);
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? RVKV_OK : hip_fail(op, e);
 }

@@ -139,8 +139,8 @@ class HipKvStorage:
     default) or, with dtype=torch.float32, f32 like rvllm's own cache (every
     operation). On an f32 pool, at head_dim 32/64/128/256 with power-of-two
     blocks, decode runs the tuned decode_f32_kernel (split partials and a
-    reduction, as on f16) and prefill the f32 matrix cores; attn_prep, and
-    prefill and decode at other shapes, run the generic kernels."""
+    reduction, as on f16), prefill the f32 matrix cores and attn_prep its f16
+    pools' kernel; other shapes run the generic kernels."""
 
     def __init__(self, n_layers: int, num_blocks: int, block_size: int,
                  n_kv_heads: int, head_dim: int, stream=None,

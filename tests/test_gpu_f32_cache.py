@@ -307,3 +307,24 @@ def test_f32_prefill_inf_value(hd):
         assert torch.isinf(out[0, key:, :, hd // 2]).all()
         out[0, key:, :, hd // 2] = want[0, key:, :, hd // 2].float()
         assert (out - want).abs().max() < 2e-5
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
+def test_f32_attn_prep_equals_f16_pool(hd):
+    """attn_prep into an f32 pool: q bit for bit as on an f16 pool, whose
+    cells are the f32 pool's rounded (one kernel, two cell types)."""
+    rows, H, KV, nb = 37, 6, 2, 5
+    g = torch.Generator("cuda").manual_seed(hd)
+    rnd = lambda *s: torch.randn(*s, device="cuda", generator=g)
+    qkv, bias = rnd(rows, (H + 2 * KV) * hd), rnd((H + 2 * KV) * hd)
+    qn, kn, c, s = rnd(hd), rnd(hd), rnd(rows, hd // 2), rnd(rows, hd // 2)
+    at = np.random.default_rng(hd).permutation(nb * 16)[:rows]
+    out = []
+    for dt in (torch.float32, torch.float16):
+        st = HipKvStorage(1, nb, 16, KV, hd, dtype=dt)
+        q = st.attn_prep_qkv(0, qkv, H, c, s, dev_u32(at // 16),
+                             dev_u32(at % 16), bias=bias, q_norm=qn, k_norm=kn)
+        ids = dev_u32(np.arange(nb))
+        out.append([q] + [st.read_blocks(0, w, ids).half() for w in (0, 1)])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)

@@ -1730,15 +1730,20 @@ void split_prefill(rvkv_pool *pool, PrefillArgs &a, uint32_t n_wg) {
 
 // Waves per workgroup: 4 at head_dim 128 with the tiles staged by LDS DMA,
 // two workgroups per CU (1.5-2 % faster than one 8-wave workgroup with
-// register staging, which is what fits without DMA); 8 at 256 (four
-// pairs); 4 at 64, where 8-wave workgroups would cost the third resident
-// wave per SIMD (measured ~7 % slower), and at 32. RVKV_PREFILL_WAVES=4|8
-// overrides at 64 and 128.
-uint32_t prefill_waves(uint32_t hd) {
+// register staging, which is what fits without DMA); 4 at 64, where 8-wave
+// workgroups would cost the third resident wave per SIMD (measured ~7 %
+// slower), and at 32. At 256 one workgroup fits a CU: 8 (four pairs, 128
+// rows), or two pairs where that still leaves one workgroup a CU, whose steps
+// are shorter (gemma-3 heads, a kernel a layer: 1000 rows under a window of
+// 512, 32 tiles of 128 rows cut in four, 24.2 -> 18.4 us; 4000 rows, 125
+// tiles, 45.6 -> 39.4; 192 tiles, two generations of the smaller ones, 47.0
+// -> 65.9). RVKV_PREFILL_WAVES=4|8 overrides at 64 and 128. tiles128: the
+// launch's query tiles of 128 rows.
+uint32_t prefill_waves(uint32_t hd, uint64_t tiles128) {
   static const char *env = getenv("RVKV_PREFILL_WAVES");
   static const uint32_t forced = env ? (uint32_t)atoi(env) : 0u;
   if (hd == 128) return forced == 8 ? 8u : 4u;
-  if (split_dims((int)hd)) return 8u;  // (four pairs)
+  if (split_dims((int)hd)) return tiles128 <= 128 ? 4u : 8u;
   if (hd == 64 && (forced == 4 || forced == 8)) return forced;
   return 4u;
 }
@@ -1806,7 +1811,8 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
   while ((1u << lg) < bs) ++lg;
   a.bs_log2 = lg;
   a.rows = (uint32_t)rows;
-  const uint32_t waves = prefill_waves(hd);
+  const uint32_t waves = prefill_waves(
+      hd, (rows + 127) / 128 * pool->n_kv * batch);
   const uint32_t bm =
       pool->f32() ? kF32Rows
                   : kWaveRows * (split_dims((int)hd) ? waves / 2 : waves);
@@ -1840,7 +1846,10 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
       if (waves == 4) launch_prefill<128, 4>(a, grid, pool->stream);
       else launch_prefill<128, 8>(a, grid, pool->stream);
       break;
-    default: launch_prefill<256, 8>(a, grid, pool->stream); break;
+    default:
+      if (waves == 4) launch_prefill<256, 4>(a, grid, pool->stream);
+      else launch_prefill<256, 8>(a, grid, pool->stream);
+      break;
   }
   hipError_t e = hipGetLastError();
   return e == hipSuccess ? RVKV_OK : hip_fail(op, e);

@@ -1831,6 +1831,23 @@ def test_prefill_cut_keys(G, hd, bs, Q, prior, window):
     assert (out - want).abs().max() < ATOL
 
 
+@pytest.mark.parametrize("Q,window", [(2048, 0), (2049, 0), (2049, 300),
+                                      (61, 0), (64, 20), (65, 0)])
+def test_prefill_hd256_workgroups(Q, window):
+    """head_dim 256 with two and with four wave pairs a workgroup (up to 128
+    tiles of 128 rows, and from there), whole and partial last row tiles."""
+    nkv, H, bs = 2, 8, 16
+    nb = -(-Q // bs)
+    st = HipKvStorage(1, nb, bs, nkv, 256)
+    fill_layer(st, 0, seed=Q)
+    table = np.random.default_rng(Q).permutation(nb).astype(np.uint32)[None]
+    q = torch.randn(1, Q, H, 256, device="cuda")
+    out = st.paged_prefill(0, q, dev_u32(table), dev_u32([0]), dev_u32([Q]),
+                           window=window)
+    want = _prefill_f64(st, q, table, [0], [Q], window)
+    assert (out - want).abs().max() < ATOL
+
+
 def test_prefill_cut_keys_streams():
     """Calls queued on three streams at once: the first two get a scratch
     region each, the third runs uncut; none disturbs another's partials."""

@@ -312,8 +312,9 @@ int rvkv_attn_prep(rvkv_pool *pool, uint32_t layer, const float *q_in,
  * arithmetic. Allocates nothing. Calls whose query rows alone leave the GPU
  * idle are cut along the keys and merged by a second launch; the partial
  * results go to the pool's scratch, half of which the first two streams that
- * such calls run on get each. On further streams, and under graph capture,
- * the keys are not cut (the same result to within rounding). */
+ * such calls run on get each. On further streams, on hipStreamPerThread and
+ * under graph capture the keys are not cut (the same result to within
+ * rounding). */
 int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
                        const uint32_t *block_tables,
                        const uint32_t *pos_offset,

@@ -43,8 +43,9 @@ namespace rvkv_detail {
 constexpr size_t kSplitBytes = (size_t)16 << 20;
 constexpr uint32_t kSplitStreams = 2;
 // The scratch region of the pool's current stream; NULL when every region
-// belongs to another stream, or while the stream is captured (a graph may be
-// replayed beside any later call): the caller then does without.
+// belongs to another stream, on hipStreamPerThread, or while the stream is
+// captured (a graph may be replayed beside any later call): the caller then
+// does without.
 void *split_scratch(rvkv_pool *pool);
 // Records "<op>: <reason>" as the last error and returns code.
 int fail(int code, const char *op, const char *reason);

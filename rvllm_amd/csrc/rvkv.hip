@@ -39,6 +39,8 @@ int hip_fail(const char *op, hipError_t e) {
 
 void *split_scratch(rvkv_pool *pool) {
   if (!pool->split_base) return nullptr;
+  // (one handle, a stream of its own in every thread: no region's owner)
+  if (pool->stream == hipStreamPerThread) return nullptr;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(pool->stream, &cs) != hipSuccess) {
     (void)hipGetLastError();

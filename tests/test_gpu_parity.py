@@ -1870,6 +1870,28 @@ def test_prefill_cut_keys_streams():
         assert (o - w).abs().max() < ATOL
 
 
+def test_prefill_per_thread_stream_is_not_cut():
+    """hipStreamPerThread (handle 2) is another stream in each host thread:
+    it owns no scratch region, so the next two streams still get theirs, and
+    its result is the one a stream without a region gets, bit for bit."""
+    st = HipKvStorage(1, 260, 16, 2, 64)
+    fill_layer(st, 0, seed=9)
+    table = np.random.default_rng(9).permutation(260)[:256].astype(np.uint32)
+    t, p, r = dev_u32(table[None]), dev_u32([4000]), dev_u32([4040])
+    q = torch.randn(1, 40, 8, 64, device="cuda")
+    outs = [torch.empty_like(q) for _ in range(4)]
+    own = st.stream
+    torch.cuda.synchronize()
+    for o, s in zip(outs, [torch.cuda.ExternalStream(2)] +
+                    [torch.cuda.Stream() for _ in range(3)]):
+        st.set_stream(s)
+        st.paged_prefill(0, q, t, p, r, out=o)
+    torch.cuda.synchronize()
+    st.set_stream(own)
+    assert torch.equal(outs[0], outs[3]) and torch.equal(outs[1], outs[2])
+    assert not torch.equal(outs[0], outs[1])  # (the second is cut)
+
+
 def test_prefill_full_prompt_from_empty():
     """Whole-prompt prefill (pos_offset 0, read_num = q_len), the
     reference's first forward of a sequence, at 1000 tokens."""

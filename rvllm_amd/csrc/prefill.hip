@@ -564,7 +564,22 @@ __global__ void __launch_bounds__(
   for (int t = 0; t < DT; ++t)
 #pragma unroll
     for (int j = 0; j < 16; ++j) o[t][j] = 0.f;
-  float m = kNegBig, l = 0.f;
+  // RELATIVE: the S products start from -m, the row's reference max (0 until
+  // the row has seen a key), in 16 registers, so scores come out of the
+  // matrix cores relative to it and the 32 subtractions a lane and tile fall
+  // away: these kernels are bound by issue, a tile costing its matrix cycles
+  // plus its vector cycles (Llama-3.2-1B heads, 6 x 2000 rows 182 -> 173 us,
+  // 300 rows behind 7700 keys 44.7 -> 42.7; Qwen3-0.6B heads, 4 x 1999 140 ->
+  // 134, a layer each). Not at head_dim 32 (the registers cost a wave a
+  // SIMD), nor for wave pairs and decodes, which other work bounds
+  // (gemma-3 heads 18.4 -> 18.7 us, 64 x 2048 decode 48.9 both). thr: what a
+  // tile's largest score has to exceed for m to move, kNegBig until the
+  // row's first key.
+  constexpr bool RELATIVE = WAVES > 1 && !SPLIT && HD >= 64;
+  float m = RELATIVE ? 0.f : kNegBig, thr = kNegBig, l = 0.f;
+  f32x16 neg_m;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) neg_m[j] = 0.f;
 
   // K row this lane feeds to the S product: sigma(ln), see the header.
   const int sig = 16 * (ln >> 4) + 8 * ((ln >> 2) & 1) + 4 * ((ln >> 3) & 1) +
@@ -889,9 +904,7 @@ __global__ void __launch_bounds__(
 
     f32x16 s[NT];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) s[t][j] = 0.f;
+    for (int t = 0; t < NT; ++t) s[t] = neg_m;
     // The two sub-tiles' accumulation chains alternate, so each MFMA's
     // dependency on the previous one of its chain is hidden.
     if (active) {
@@ -994,12 +1007,25 @@ __global__ void __launch_bounds__(
     // exceeds it by more than 2^8, so probabilities stay <= 256 (exact
     // in f16's range) and O and l are rescaled on few tiles; the final
     // division by l cancels whichever m was used.
-    const bool grow = mx > m + 8.0f;
+    const bool grow = RELATIVE ? mx > thr : mx > m + 8.0f;
     if (__builtin_amdgcn_ballot_w64(grow) != 0) {
-      const float m_new = grow ? mx : m;
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+      const float m_new = grow ? (RELATIVE ? m + mx : mx) : m;
+      const float d = m_new - m;
+      // (RELATIVE: a row's first keys may lie below 0, where there is
+      // nothing to rescale yet)
+      const float alpha =
+          __builtin_amdgcn_exp2f(RELATIVE ? -fmaxf(d, 0.f) : -d);
       m = m_new;
       l *= alpha;
+      if constexpr (RELATIVE) {
+        thr = grow ? 8.0f : thr;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) neg_m[j] = -m;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) s[t][j] -= d;
+      }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
@@ -1014,7 +1040,8 @@ __global__ void __launch_bounds__(
       for (int c = 0; c < 2; ++c) {
 #pragma unroll
         for (int e = 0; e < 8; ++e)
-          pb[t][c][e] = (_Float16)__builtin_amdgcn_exp2f(s[t][8 * c + e] - m);
+          pb[t][c][e] = (_Float16)__builtin_amdgcn_exp2f(
+              RELATIVE ? s[t][8 * c + e] : s[t][8 * c + e] - m);
 #pragma unroll
         for (int e = 0; e < 8; e += 2)
           psum = __builtin_amdgcn_fdot2(h2{pb[t][c][e], pb[t][c][e + 1]},
@@ -1105,6 +1132,7 @@ __global__ void __launch_bounds__(
     kt += BN;
   }
 
+  if (RELATIVE && thr != 8.0f) m = kNegBig;  // no key seen
   if constexpr (WAVES == 1) {
     if (newtok != 0xFFFFFFFFu && tid < CPR) {
       const uint32_t nb = a.new_blk[b], no = a.new_off[b];

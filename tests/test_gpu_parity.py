@@ -1702,6 +1702,31 @@ def test_prefill_large_scores(hd):
     assert np.isfinite(out).all() and np.abs(out - want).max() < ATOL
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("prior", [[2500, 70], [0, 0]])  # keys cut, or not
+def test_prefill_scores_far_from_zero(hd, prior):
+    """Scores all near -460 or all near +460 (log2 units), with a step up
+    part of the way: the row's reference max starts below zero, and moves.
+    (Bound: f16 probabilities 2^-11 and 460 * 2^-22 of the scores' rounding,
+    times |v| < 5, stay under 2e-3.)"""
+    Q, nkv, bs = 200, 2, 16
+    mb = -(-(max(prior) + Q) // bs)
+    st = HipKvStorage(1, 2 * mb, bs, nkv, hd)
+    at = torch.arange(2 * mb * bs, device="cuda")
+    k = torch.randn(len(at), nkv, hd, device="cuda") * 0.2 - 320 / hd ** 0.5
+    k[: mb * bs][(at[: mb * bs] > 100) & (at[: mb * bs] < 130)] += 12 / hd ** 0.5
+    k[mb * bs:] *= -1
+    st.write_tokens(0, (at // bs).int(), (at % bs).int(), k,
+                    torch.randn(len(at), nkv, hd, device="cuda"))
+    q = 1 + 0.05 * torch.randn(2, Q, 2 * nkv, hd, device="cuda")
+    tables = np.arange(2 * mb, dtype=np.uint32).reshape(2, mb)
+    read = [x + Q for x in prior]
+    out = st.paged_prefill(0, q, dev_u32(tables), dev_u32(prior),
+                           dev_u32(read))
+    want = _prefill_f64(st, q, tables, prior, read, 0)
+    assert (out - want).abs().max() < ATOL
+
+
 @pytest.mark.parametrize("hd,G,batch,ctx,dtype", [
     (64, 3, 8, 512, torch.float32),     # one partition of 16 waves
     (64, 2, 1, 33, torch.float16),      # fewer chunks than waves

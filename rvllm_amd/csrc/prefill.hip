@@ -568,9 +568,9 @@ __global__ void __launch_bounds__(
   // the row has seen a key), in 16 registers, so scores come out of the
   // matrix cores relative to it and the 32 subtractions a lane and tile fall
   // away: these kernels are bound by issue, a tile costing its matrix cycles
-  // plus its vector cycles (Llama-3.2-1B heads, 6 x 2000 rows 182 -> 173 us,
-  // 300 rows behind 7700 keys 44.7 -> 42.7; Qwen3-0.6B heads, 4 x 1999 140 ->
-  // 134, a layer each). Not at head_dim 32 (the registers cost a wave a
+  // plus its vector cycles (Llama-3.2-1B heads, 6 x 2000 rows 179 -> 173 us,
+  // 300 rows behind 7700 keys 44.7 -> 42.1; Qwen3-0.6B heads, 4 x 1999 140 ->
+  // 136, a layer each). Not at head_dim 32 (the registers cost a wave a
   // SIMD), nor for wave pairs and decodes, which other work bounds
   // (gemma-3 heads 18.4 -> 18.7 us, 64 x 2048 decode 48.9 both). thr: what a
   // tile's largest score has to exceed for m to move, kNegBig until the

@@ -1805,12 +1805,14 @@ int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
     return fail(RVKV_EINVAL, op, "scale must be positive and finite");
   // The matrix-core kernels take head_dim 32/64/128/256 and power-of-two
   // blocks, of >= 8 tokens (f16 cells) or >= 4 (f32 cells, whose batch and
-  // q_len stay bounded as in the generic kernel); every other shape runs the
-  // generic kernel.
+  // q_len stay bounded as in the generic kernel) that their 32-bit offsets
+  // inside a block reach (f16: the whole block, f32: one head of it); every
+  // other shape runs the generic kernel.
   if ((hd != 32 && hd != 64 && hd != 128 && hd != 256) ||
       bs < (pool->f32() ? 4u : 8u) || (bs & (bs - 1)) != 0 ||
       (uint64_t)max_blocks * bs > 0x80000000ull ||
-      (pool->f32() ? batch > 65535 || q_len > 65535
+      (pool->f32() ? batch > 65535 || q_len > 65535 ||
+                         (uint64_t)bs * hd * 4 >= 0x100000000ull
                    : pool->block_elems * 2 >= 0x100000000ull))
     return rvkv_detail::generic_attention(
         op, pool, layer, q, block_tables, max_blocks, pos_offset,

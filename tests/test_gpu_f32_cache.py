@@ -328,3 +328,25 @@ def test_f32_attn_prep_equals_f16_pool(hd):
         out.append([q] + [st.read_blocks(0, w, ids).half() for w in (0, 1)])
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+def test_f32_prefill_block_past_32_bit_rows():
+    """One block of 2^23 tokens at head_dim 256 (8 GiB of K, 8 of V): a row's
+    byte offset in its block passes 2^32 from token 2^22 on. Rows and keys
+    there against float64; every product and sum is f32: 2e-5."""
+    bs, hd, Q, window = 1 << 23, 256, 40, 70
+    p0 = (1 << 22) + 1000
+    st = HipKvStorage(1, 1, bs, 1, hd, dtype=torch.float32)
+    n = window + Q
+    pos = np.arange(p0 - window, p0 + Q)
+    k, v = (torch.randn(n, 1, hd, device="cuda") for _ in range(2))
+    st.write_tokens(0, dev_u32(0 * pos), dev_u32(pos), k, v)
+    q = torch.randn(1, Q, 2, hd, device="cuda")
+    out = st.paged_prefill(0, q, dev_u32([[0]]), dev_u32([p0]),
+                           dev_u32([p0 + Q]), window=window)
+    j, i = torch.arange(n, device="cuda"), torch.arange(Q, device="cuda")
+    see = (j[None] <= i[:, None] + window) & (j[None] > i[:, None])
+    s = torch.einsum("qhd,kd->hqk", q[0].double(), k[:, 0].double())
+    s = (s / hd ** 0.5).masked_fill(~see, -torch.inf)
+    want = (torch.softmax(s, -1) @ v[:, 0].double()).transpose(0, 1)
+    assert (out[0] - want).abs().max() < 2e-5

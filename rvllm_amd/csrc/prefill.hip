@@ -1588,7 +1588,9 @@ __global__ void __launch_bounds__(64 * kF32Waves, HD <= 64 ? 2 : 1)
 // of a q row (token, head), four elements each; weights 2^(m_i - M). Rows of
 // uncut tiles are left alone (the prefill kernel wrote them). Bound by the
 // launch and the round trips to the partials: eight pieces' (m, l) and
-// partials are loaded at a time.
+// partials are loaded at a time. A piece of weight 0 (no key seen, or scores
+// too low) stays out of the sums, so an inf in it meets no 0; l = NaN is a
+// piece that was seen, and L makes the row NaN.
 template <int HD, int BM, int BN>
 __global__ void __launch_bounds__(256)
     prefill_reduce_kernel(PrefillArgs a, uint32_t n_rows) {
@@ -1621,28 +1623,27 @@ __global__ void __launch_bounds__(256)
     float mx = M;
 #pragma unroll
     for (int k = 0; k < 8; ++k)
-      if (x[k].y > 0.f) mx = fmaxf(mx, x[k].x);
+      if (x[k].y != 0.f) mx = fmaxf(mx, x[k].x);
     const float corr = __builtin_amdgcn_exp2f(M - mx);
     M = mx;
     L *= corr;
-    acc.x *= corr;
-    acc.y *= corr;
-    acc.z *= corr;
-    acc.w *= corr;
+    acc.x = corr != 0.f ? acc.x * corr : 0.f;
+    acc.y = corr != 0.f ? acc.y * corr : 0.f;
+    acc.z = corr != 0.f ? acc.z * corr : 0.f;
+    acc.w = corr != 0.f ? acc.w * corr : 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       // (l = 0: the row sees no key of the piece)
-      const float w = i + k < np && x[k].y > 0.f
-                          ? __builtin_amdgcn_exp2f(x[k].x - M)
-                          : 0.f;
-      L += x[k].y * w;
-      acc.x += v[k].x * w;
-      acc.y += v[k].y * w;
-      acc.z += v[k].z * w;
-      acc.w += v[k].w * w;
+      const bool live = i + k < np && x[k].y != 0.f;
+      const float w = live ? __builtin_amdgcn_exp2f(x[k].x - M) : 0.f;
+      L += live ? x[k].y * w : 0.f;
+      acc.x += w != 0.f ? v[k].x * w : 0.f;
+      acc.y += w != 0.f ? v[k].y * w : 0.f;
+      acc.z += w != 0.f ? v[k].z * w : 0.f;
+      acc.w += w != 0.f ? v[k].w * w : 0.f;
     }
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  const float inv = L != 0.f ? 1.0f / L : 0.f;
   *reinterpret_cast<float4 *>(a.out + at) =
       make_float4(acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv);
 }

@@ -1917,6 +1917,96 @@ def test_prefill_per_thread_stream_is_not_cut():
     assert not torch.equal(outs[0], outs[1])  # (the second is cut)
 
 
+@pytest.mark.parametrize("hd", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_prefill_cut_keys_keep_nan(dtype, hd):
+    """A NaN in a query row, or an overflowed K cell, gives NaN in the rows it
+    reaches whether the keys are cut (the first two streams) or not (the
+    third): the merge of the pieces drops nothing that was seen."""
+    Q, nkv, H, bs, prior = 20, 1, 2, 16, 2700
+    n = prior + Q
+    nb = -(-n // bs)
+    table = np.random.default_rng(hd).permutation(nb).astype(np.uint32)
+    at = np.arange(n)
+    slots = dev_u32(table[at // bs]), dev_u32(at % bs)
+    t, p, r = dev_u32(table[None]), dev_u32([prior]), dev_u32([n])
+    st = HipKvStorage(1, nb, bs, nkv, hd, dtype=dtype)
+    k, v = (torch.randn(n, nkv, hd, device="cuda").to(dtype)
+            for _ in range(2))
+    q = torch.randn(1, Q, H, hd, device="cuda")
+    own, streams = st.stream, [torch.cuda.Stream() for _ in range(2)]
+
+    def both():
+        outs = []
+        torch.cuda.synchronize()
+        for s in [own] + streams:
+            st.set_stream(s)
+            outs.append(st.paged_prefill(0, q, t, p, r,
+                                         out=torch.zeros_like(q)))
+            torch.cuda.synchronize()
+        st.set_stream(own)
+        assert torch.equal(outs[0].isnan(), outs[1].isnan())
+        return outs[0], outs[2]
+
+    st.write_tokens(0, *slots, k, v)
+    cut, whole = both()
+    assert not torch.equal(cut, whole)  # (the keys are cut)
+    bad = torch.zeros(Q, H, dtype=torch.bool, device="cuda")
+    q[0, 3, 1, 5] = float("nan")
+    bad[3, 1] = True
+    for out in both():
+        assert torch.equal(out[0].isnan().all(-1), bad)
+        assert torch.equal(out[0].isnan().any(-1), bad)
+    q[0, 3, 1, 5] = 0.5
+    # an inf K cell in the first, a middle and the last piece
+    for key in (7, 1300, prior + 4):
+        kk = k.clone()
+        kk[key, 0, 2] = float("inf")
+        st.write_tokens(0, *slots, kk, v)
+        cut, whole = both()
+        assert torch.equal(cut.isnan(), whole.isnan())
+        sees = torch.arange(Q, device="cuda") + prior >= key
+        up = q[0, :, :, 2] > 0  # the score is +inf: NaN in the softmax
+        assert cut[0].isnan().all(-1)[sees[:, None] & up].all()
+        assert not cut[0].isnan().any(-1)[~sees].any()
+
+
+@pytest.mark.parametrize("hd", [64, 256])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_prefill_cut_keys_inf_value(dtype, hd):
+    """An inf in V reaches the rows that see its key as an inf, and leaves the
+    others finite, wherever its piece of the cut keys lies (11 pieces: the
+    merge loads eight at a time, the last ones again past the end)."""
+    Q, nkv, H, bs, prior = 20, 1, 2, 16, 2700
+    n = prior + Q
+    nb = -(-n // bs)
+    table = np.random.default_rng(hd).permutation(nb).astype(np.uint32)
+    at = np.arange(n)
+    slots = dev_u32(table[at // bs]), dev_u32(at % bs)
+    t, p, r = dev_u32(table[None]), dev_u32([prior]), dev_u32([n])
+    st = HipKvStorage(1, nb, bs, nkv, hd, dtype=dtype)
+    k, v = (torch.randn(n, nkv, hd, device="cuda").to(dtype)
+            for _ in range(2))
+    q = torch.randn(1, Q, H, hd, device="cuda")
+    st.write_tokens(0, *slots, k, v)
+    want = _prefill_f64(st, q, table[None], [prior], [n], 0)
+    tol = 2e-5 if dtype == torch.float32 else ATOL
+    # (f16 cells: keys that every row sees; the f16 products give a NaN to the
+    # rows of a tile that do not see an inf key, cut or not)
+    seen_by_some = (prior + 4, n - 1) if dtype == torch.float32 else ()
+    for key in (7, 1300, 2650) + seen_by_some:
+        vv = v.clone()
+        vv[key, 0, hd // 2] = float("inf")
+        st.write_tokens(0, *slots, k, vv)
+        out = st.paged_prefill(0, q, t, p, r)
+        sees = torch.arange(Q, device="cuda") + prior >= key
+        at_d = out[0, :, :, hd // 2]
+        assert torch.equal(torch.isinf(at_d), sees[:, None].expand(Q, H))
+        out[0, :, :, hd // 2] = torch.where(
+            sees[:, None], want[0, :, :, hd // 2].float(), at_d)
+        assert (out - want).abs().max() < tol
+
+
 def test_prefill_full_prompt_from_empty():
     """Whole-prompt prefill (pos_offset 0, read_num = q_len), the
     reference's first forward of a sequence, at 1000 tokens."""

@@ -1610,8 +1610,9 @@ __global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, true))
 // Reduction pass (only for sequences split over several partitions): one
 // workgroup per (sequence, query head) merges its partitions: M = max m_i,
 // out = sum_i 2^(m_i - M) acc_i / sum_i 2^(m_i - M) l_i. Partitions that saw
-// no visible key carry l = 0 and are skipped. Bound by the launch and its
-// round trips to memory: a wave loads eight partitions' (m, l) and partials
+// no visible key carry l = 0 and are skipped; any of weight 0 stays out of the
+// sums, so an inf in it meets no 0. Bound by the launch and its round trips to
+// memory: a wave loads eight partitions' (m, l) and partials
 // at once, and with more than eight partitions four waves share them, merged
 // through LDS (25 partitions of Qwen3-0.6B heads:
 // 4.8 -> 4.0 us).
@@ -1675,7 +1676,7 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(
     M = mx;
     L *= corr;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] *= corr;
+    for (int e = 0; e < EPL; ++e) acc[e] = corr != 0.f ? acc[e] * corr : 0.f;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       // (l = 0: a partition that saw no visible key stays out)
@@ -1706,10 +1707,11 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(
 #pragma unroll
       for (int e = 0; e < EPL; ++e)
         if (lane * EPL + e < HD)
-          acc[e] = acc[e] * ca + red_s[w][lane * EPL + e] * cb;
+          acc[e] = (ca != 0.f ? acc[e] * ca : 0.f) +
+                   (cb != 0.f ? red_s[w][lane * EPL + e] * cb : 0.f);
     }
   }
-  const float inv = L > 0.f ? 1.0f / L : 0.f;
+  const float inv = L != 0.f ? 1.0f / L : 0.f;
 #pragma unroll
   for (int e = 0; e < EPL; ++e) {
     const int d = lane * EPL + e;

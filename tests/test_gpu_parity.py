@@ -1777,6 +1777,40 @@ def test_decode_partition_rule(hd, G, batch, ctx, dtype):
         assert (out - want[:, 0]).abs().max() < tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("ctx", [9000, 15000])
+def test_decode_reduction_leaves_out_weightless_partials(dtype, ctx):
+    """More than eight partitions, some of them with only keys of a score so
+    low that their weight in the merge is 0, and an inf among their values:
+    it stays out, also where such partitions are all that the merge loads at
+    once (eight) or all that one of its waves has (a quarter)."""
+    hd, bs, P = 128, 16, 256
+    nb = -(-ctx // bs)
+    table = np.arange(nb, dtype=np.uint32)[::-1].copy()
+    at = np.arange(ctx)
+    slots = dev_u32(table[at // bs]), dev_u32(at % bs)
+    st = HipKvStorage(1, nb, bs, 1, hd, dtype=dtype)
+    t, n = dev_u32(table[None]), dev_u32([ctx])
+    assert st.decode_partition_tokens(1, 2, ctx) == P
+    parts = -(-ctx // P)
+    per = -(-parts // 4)
+    q = 1 + 0.1 * torch.randn(1, 2, hd, device="cuda")
+    tol = 2e-5 if dtype == torch.float32 else ATOL
+    for a, b in ((0, 1), (0, 8), (0, per), (per, 2 * per), (per, per + 8),
+                 (3 * per, parts), (8, parts), (0, parts - 1)):
+        low = slice(a * P, min(b * P, ctx))
+        k, v = (torch.randn(ctx, 1, hd, device="cuda").to(dtype)
+                for _ in range(2))
+        k[low] = -350 / hd ** 0.5
+        v[low] = 0
+        st.write_tokens(0, *slots, k, v)
+        want = _prefill_f64(st, q[:, None], table[None], [ctx - 1], [ctx], 0)
+        v[low, 0, 3] = float("inf")
+        st.write_tokens(0, *slots, k, v)
+        out = st.paged_decode(0, q, t, n, ctx)
+        assert (out - want[:, 0]).abs().max() < tol, (a, b)
+
+
 def _prefill_f64(st, q, tables, prior, read, window):
     """Prefill attention in float64 from the raw cache (keys behind an
     out-of-range id hidden), on the GPU."""

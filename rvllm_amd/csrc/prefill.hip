@@ -224,6 +224,14 @@ struct Lds {
 __device__ __forceinline__ float vmax3(float a, float b, float c) {
   return __builtin_fmaxf(__builtin_fmaxf(a, b), c);
 }
+__device__ __forceinline__ float vmin3(float a, float b, float c) {
+  return __builtin_fminf(__builtin_fminf(a, b), c);
+}
+
+// a * b, and 0 where a or b is 0 whatever the other is (v_mul_legacy_f32): a
+// weight of 0 takes an inf or a NaN out of a sum at the cost of a product.
+extern "C" __device__ __attribute__((const)) float rvkv_mul0(
+    float a, float b) __asm("llvm.amdgcn.fmul.legacy");
 
 // Lanes i and i ^ 32 combined: v_permlane32_swap of v with itself leaves
 // the lower half's value in element 0 and the upper half's in element 1 of
@@ -1450,29 +1458,40 @@ __global__ void __launch_bounds__(64 * kF32Waves, HD <= 64 ? 2 : 1)
         }
       }
     }
-    float mx = m;
+    float mx = m, mn = s[0];
 #pragma unroll
-    for (int j = 0; j < 16; j += 2) mx = vmax3(mx, s[j], s[j + 1]);
+    for (int j = 0; j < 16; j += 2) {
+      mx = vmax3(mx, s[j], s[j + 1]);
+      mn = vmin3(mn, s[j], s[j + 1]);
+    }
     mx = max_halves(mx);
     if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {
       const float alpha = __builtin_amdgcn_exp2f(m - mx);
       m = mx;
       l *= alpha;
+      // (weight 0: what was summed stays out, an inf too)
 #pragma unroll
       for (int t = 0; t < DT; ++t)
 #pragma unroll
-        for (int j = 0; j < 16; ++j) o[t][j] *= alpha;
+        for (int j = 0; j < 16; ++j)
+          o[t][j] = rvkv_mul0(o[t][j], alpha);
     }
+    // (2^-126 is the smallest weight; found from the scores, beside their
+    // maximum, because a branch on the weights would hold P.V back)
+    const bool zero =
+        __builtin_amdgcn_ballot_w64(row_ok && mn - m < -126.f) != 0;
 #pragma unroll
     for (int j = 0; j < 16; ++j) {
       s[j] = __builtin_amdgcn_exp2f(s[j] - m);
       l += s[j];
     }
-    // In a tile that some rows see only in part, a V that is not finite must
-    // not meet another row's zero weight (0 * inf): it is left out of the
-    // product and added row by row afterwards.
+    // Where a weight is 0 (a tile that some rows see only in part, a score
+    // too low), a V that is not finite must not meet it (0 * inf): it is left
+    // out of the product and added row by row afterwards. (Keeping such V out
+    // here and where states merge costs 1.5 %: 700 rows of SmolLM2 heads
+    // 35.2 -> 35.7 us a layer with attn_prep; as selects it was 10 %.)
     bool by_row = false;
-    if (!whole) {
+    if (zero) {
       bool odd = false;
 #pragma unroll
       for (int j = 0; j < 16; ++j)
@@ -1559,14 +1578,15 @@ __global__ void __launch_bounds__(64 * kF32Waves, HD <= 64 ? 2 : 1)
     for (int t = 0; t < DT; ++t)
 #pragma unroll
       for (int j = 0; j < 16; ++j)
-        o[t][j] = o[t][j] * aw + src[(2 + t * 16 + j) * 64] * bw;
+        o[t][j] = rvkv_mul0(o[t][j], aw) +
+                  rvkv_mul0(src[(2 + t * 16 + j) * 64], bw);
     m = M;
   }
   if (!row_ok) return;
   const size_t idx =
       partial ? (size_t)wi.piece * a.batch * a.q_len * a.n_heads + qrow : qrow;
   float *op = (partial ? a.ws_acc : a.out) + idx * HD;
-  const float inv = partial ? 1.f : (l > 0.f ? 1.0f / l : 0.f);
+  const float inv = partial ? 1.f : (l != 0.f ? 1.0f / l : 0.f);
 #pragma unroll
   for (int g = 0; g < 4; ++g)
 #pragma unroll

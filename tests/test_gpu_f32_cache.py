@@ -350,3 +350,39 @@ def test_f32_prefill_block_past_32_bit_rows():
     s = (s / hd ** 0.5).masked_fill(~see, -torch.inf)
     want = (torch.softmax(s, -1) @ v[:, 0].double()).transpose(0, 1)
     assert (out[0] - want).abs().max() < 2e-5
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
+@pytest.mark.parametrize("prior", [100, 1900])  # keys whole, and cut
+def test_f32_prefill_inf_value_without_weight(hd, prior):
+    """A V row that is not finite, behind a score so low that its weight is 0
+    in f32 (2^-430 and less), stays out of every row: single keys anywhere in
+    a key tile, and a run of them that fills a tile, which is all that some
+    wave or piece has seen by then."""
+    Q, bs = 40, 16
+    n = prior + Q
+    nb = -(-n // bs)
+    table = np.random.default_rng(hd).permutation(nb).astype(np.uint32)
+    at = np.arange(n)
+    slots = dev_u32(table[at // bs]), dev_u32(at % bs)
+    st = HipKvStorage(1, nb, bs, 1, hd, dtype=torch.float32)
+    q = 1 + 0.1 * torch.randn(1, Q, 2, hd, device="cuda")
+    for keys in ([0], [31], [64], [prior - 5], list(range(40)),
+                 list(range(64, 96)), list(range(prior - 40, prior))):
+        k, v = (torch.randn(n, 1, hd, device="cuda") for _ in range(2))
+        k[keys] = -350 / hd ** 0.5  # (score ~ -350; the others within +-6)
+        v[keys] = 0
+        st.write_tokens(0, *slots, k, v)
+        # (float64 weights of those keys are 1e-140: v = 0 there is the same)
+        want = _prefill_f64_of(st, q, table, prior, n)
+        v[keys, 0, 3] = float("inf")
+        v[keys, 0, hd - 1] = float("nan")
+        st.write_tokens(0, *slots, k, v)
+        out = st.paged_prefill(0, q, dev_u32(table[None]), dev_u32([prior]),
+                               dev_u32([n]))
+        assert (out - want).abs().max() < 2e-5, keys[0]
+
+
+def _prefill_f64_of(st, q, table, prior, n):
+    from tests.test_gpu_parity import _prefill_f64
+    return _prefill_f64(st, q, table[None], [prior], [n], 0)

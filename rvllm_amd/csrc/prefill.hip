@@ -281,6 +281,14 @@ __device__ __forceinline__ uint32_t lo_bound(uint32_t p, int32_t window) {
                                                   : 0u;
 }
 
+// Position of sequence b's first query row in a prefill, held where no row's
+// position passes 2^32 (tables end at 2^31 keys: such rows see the same).
+__device__ __forceinline__ uint32_t first_pos(const PrefillArgs &a,
+                                              uint32_t b) {
+  typedef const __attribute__((address_space(4))) uint32_t cu32;
+  return min(*(cu32 *)(uintptr_t)(a.pos_offset + b), ~a.q_len);
+}
+
 // The keys [begin, end) that the rows of query tile `tile` of sequence b see
 // in a prefill, begin on a key-tile boundary; shared by the prefill kernel
 // and its reduction, which must agree on a tile's pieces.
@@ -456,8 +464,7 @@ __global__ void __launch_bounds__(
                           ? min(*(cu32s *)(uintptr_t)(a.read_num + b),
                                 a.dec_ctx_cap)
                           : *(cu32s *)(uintptr_t)(a.read_num + b);
-  const uint32_t off =
-      DEC ? rn - 1u : *(cu32s *)(uintptr_t)(a.pos_offset + b);
+  const uint32_t off = DEC ? rn - 1u : first_pos(a, b);
   const uint32_t cap = a.max_blocks << a.bs_log2;
   const uint32_t ctx = min(rn, cap);
   if (DEC && a.dec_parts) {
@@ -1277,7 +1284,7 @@ __global__ void __launch_bounds__(64 * kF32Waves, HD <= 64 ? 2 : 1)
   typedef const __attribute__((address_space(4))) uint32_t cu32;
   const uint32_t ctx = min(*(cu32 *)(uintptr_t)(a.read_num + b),
                            a.max_blocks << a.bs_log2);
-  const uint32_t off = *(cu32 *)(uintptr_t)(a.pos_offset + b);
+  const uint32_t off = first_pos(a, b);
   const uint32_t *table = a.tables + (size_t)b * a.max_blocks;
   const uint32_t bs_mask = (1u << a.bs_log2) - 1u;
 
@@ -1622,7 +1629,7 @@ __global__ void __launch_bounds__(256)
   const uint32_t ctx = min(a.read_num[b], a.max_blocks << a.bs_log2);
   const uint32_t r = qi * a.group + head % a.group;
   const uint32_t np =
-      tile_keys_of<BM, BN>(a, a.pos_offset[b], ctx, r / BM, a.rows)
+      tile_keys_of<BM, BN>(a, first_pos(a, b), ctx, r / BM, a.rows)
           .pieces(a.split_keys);
   if (np < 2) return;
   const float2 *ml = reinterpret_cast<const float2 *>(a.ws_ml) + row;

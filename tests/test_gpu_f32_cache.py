@@ -386,3 +386,21 @@ def test_f32_prefill_inf_value_without_weight(hd, prior):
 def _prefill_f64_of(st, q, table, prior, n):
     from tests.test_gpu_parity import _prefill_f64
     return _prefill_f64(st, q, table[None], [prior], [n], 0)
+
+
+def test_f32_prefill_position_near_2_32():
+    """Positions up to 2^32 - 1 are past every key: a row there sees all of
+    them (no wrap to position 0), cut keys or whole."""
+    hd, bs, Q = 64, 16, 9
+    for n in (200, 3000):
+        nb = -(-n // bs)
+        st = HipKvStorage(1, nb, bs, 1, hd, dtype=torch.float32)
+        at = np.arange(n)
+        k, v = (torch.randn(n, 1, hd, device="cuda") for _ in range(2))
+        st.write_tokens(0, dev_u32(at // bs), dev_u32(at % bs), k, v)
+        q = torch.randn(1, Q, 2, hd, device="cuda")
+        t = dev_u32(np.arange(nb)[None])
+        want = st.paged_prefill(0, q, t, dev_u32([n]), dev_u32([n]))
+        for off in (2 ** 32 - 1, 2 ** 32 - 5, 2 ** 31):
+            out = st.paged_prefill(0, q, t, dev_u32([off]), dev_u32([n]))
+            assert torch.equal(out, want), off

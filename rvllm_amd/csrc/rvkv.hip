@@ -1853,7 +1853,8 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
   if (one_workgroup(p, decode_rate(p, n_heads, gt), max_ctx, P,
                     0.4 * max_ctx * pairs))
     P = std::max<uint64_t>(P, ((uint64_t)max_ctx + 63) / 64 * 64);
-  return (uint32_t)P;
+  // (a bound near 2^32, "none", must not round up to 0 in 32 bits)
+  return (uint32_t)std::min<uint64_t>(P, 1u << 30);
 }
 
 // Short items: even the longest workgroup has under 192 context tokens.

@@ -1777,6 +1777,36 @@ def test_decode_partition_rule(hd, G, batch, ctx, dtype):
         assert (out - want[:, 0]).abs().max() < tol
 
 
+@pytest.mark.parametrize("hd,nkv,G,dtype", [
+    (128, 8, 2, torch.float16), (256, 1, 4, torch.float32),
+    (256, 2, 8, torch.float16), (64, 5, 3, torch.float32)])
+def test_decode_unbounded_max_ctx_len(hd, nkv, G, dtype):
+    """max_ctx_len up to 2^32 - 1 (no bound): partitions of a size above 0 for
+    every batch, and the result of the exact bound."""
+    bs, H = 16, nkv * G
+    st = HipKvStorage(1, 40, bs, nkv, hd, dtype=dtype)
+    for batch in (1, 30, 240, 600):
+        for top in (2 ** 31, 2 ** 32 - 64, 2 ** 32 - 63, 2 ** 32 - 1):
+            P = st.decode_partition_tokens(batch, H, top)
+            assert P > 0 and P * 520 * 32 >= top
+            st.decode_workspace_bytes(batch, H, top)
+    at = torch.arange(40 * bs, device="cuda")
+    k, v = (torch.randn(40 * bs, nkv, hd, device="cuda").to(dtype)
+            for _ in range(2))
+    st.write_tokens(0, (at // bs).int(), (at % bs).int(), k, v)
+    batch = 600
+    rng = np.random.default_rng(hd)
+    lens = rng.integers(1, 100, batch)
+    t = dev_u32(rng.integers(0, 40, (batch, 7)))
+    q = torch.randn(batch, H, hd, device="cuda")
+    want = st.paged_decode(0, q, t, dev_u32(lens), 112)
+    out = st.paged_decode(0, q, t, dev_u32(lens), 2 ** 32 - 1)
+    # (f16 cells: the weights are f16 relative to each wave's own maximum, and
+    # the launch may split a context over other waves)
+    tol = 2e-5 if dtype == torch.float32 else ATOL
+    assert (out - want).abs().max() < tol
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
 @pytest.mark.parametrize("ctx", [9000, 15000])
 def test_decode_reduction_leaves_out_weightless_partials(dtype, ctx):

@@ -84,3 +84,8 @@ int generic_attention(const char *op, const rvkv_pool *pool, uint32_t layer,
                       uint32_t q_len, uint32_t n_heads, uint32_t ctx_cap,
                       float scale, int32_t window, float *out);
 }  // namespace rvkv_detail
+
+// a * b, and 0 where a or b is 0 whatever the other is (v_mul_legacy_f32): a
+// weight of 0 takes an inf or a NaN out of a sum at the cost of a product.
+extern "C" __device__ __attribute__((const)) float rvkv_mul0(
+    float a, float b) __asm("llvm.amdgcn.fmul.legacy");

@@ -228,11 +228,6 @@ __device__ __forceinline__ float vmin3(float a, float b, float c) {
   return __builtin_fminf(__builtin_fminf(a, b), c);
 }
 
-// a * b, and 0 where a or b is 0 whatever the other is (v_mul_legacy_f32): a
-// weight of 0 takes an inf or a NaN out of a sum at the cost of a product.
-extern "C" __device__ __attribute__((const)) float rvkv_mul0(
-    float a, float b) __asm("llvm.amdgcn.fmul.legacy");
-
 // Lanes i and i ^ 32 combined: v_permlane32_swap of v with itself leaves
 // the lower half's value in element 0 and the upper half's in element 1 of
 // every lane, in the VALU (no LDS round trip as for a bpermute).
@@ -1654,20 +1649,20 @@ __global__ void __launch_bounds__(256)
     const float corr = __builtin_amdgcn_exp2f(M - mx);
     M = mx;
     L *= corr;
-    acc.x = corr != 0.f ? acc.x * corr : 0.f;
-    acc.y = corr != 0.f ? acc.y * corr : 0.f;
-    acc.z = corr != 0.f ? acc.z * corr : 0.f;
-    acc.w = corr != 0.f ? acc.w * corr : 0.f;
+    acc.x = rvkv_mul0(acc.x, corr);
+    acc.y = rvkv_mul0(acc.y, corr);
+    acc.z = rvkv_mul0(acc.z, corr);
+    acc.w = rvkv_mul0(acc.w, corr);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       // (l = 0: the row sees no key of the piece)
       const bool live = i + k < np && x[k].y != 0.f;
       const float w = live ? __builtin_amdgcn_exp2f(x[k].x - M) : 0.f;
       L += live ? x[k].y * w : 0.f;
-      acc.x += w != 0.f ? v[k].x * w : 0.f;
-      acc.y += w != 0.f ? v[k].y * w : 0.f;
-      acc.z += w != 0.f ? v[k].z * w : 0.f;
-      acc.w += w != 0.f ? v[k].w * w : 0.f;
+      acc.x += rvkv_mul0(v[k].x, w);
+      acc.y += rvkv_mul0(v[k].y, w);
+      acc.z += rvkv_mul0(v[k].z, w);
+      acc.w += rvkv_mul0(v[k].w, w);
     }
   }
   const float inv = L != 0.f ? 1.0f / L : 0.f;

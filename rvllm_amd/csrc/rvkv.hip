@@ -1676,7 +1676,7 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(
     M = mx;
     L *= corr;
 #pragma unroll
-    for (int e = 0; e < EPL; ++e) acc[e] = corr != 0.f ? acc[e] * corr : 0.f;
+    for (int e = 0; e < EPL; ++e) acc[e] = rvkv_mul0(acc[e], corr);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       // (l = 0: a partition that saw no visible key stays out)
@@ -1707,8 +1707,8 @@ __global__ void __launch_bounds__(256) decode_reduce_kernel(
 #pragma unroll
       for (int e = 0; e < EPL; ++e)
         if (lane * EPL + e < HD)
-          acc[e] = (ca != 0.f ? acc[e] * ca : 0.f) +
-                   (cb != 0.f ? red_s[w][lane * EPL + e] * cb : 0.f);
+          acc[e] = rvkv_mul0(acc[e], ca) +
+                   rvkv_mul0(red_s[w][lane * EPL + e], cb);
     }
   }
   const float inv = L != 0.f ? 1.0f / L : 0.f;

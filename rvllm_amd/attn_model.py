@@ -119,15 +119,17 @@ class HipBackend:
         # and 0.86 ms of a prompt's); _sent: that copy is done.
         self._stage = torch.empty(0, dtype=torch.int32)
         self._sent = torch.cuda.Event()
-        self._rope_rows(min(cfg.context_length, 4096))
+        # RoPE rows of every position the model takes, on the GPU; a forward
+        # gathers its own (computing 1700 rows' angles on the host took 0.9 ms
+        # a forward). 2^17 positions take 0.2-0.3 s here, once.
+        self._rope = self._rope_rows(np.arange(min(cfg.context_length,
+                                                   1 << 17)))
 
-    def _rope_rows(self, n: int) -> None:
-        """The RoPE table of positions 0 .. n - 1, on the GPU; a forward
-        gathers its rows (computing 1700 rows' angles on the host took
-        0.9 ms a forward)."""
-        self._rope = tuple(torch.from_numpy(a).to(self.dev) for a in
-                           rope_cos_sin(self.cfg.rope_theta,
-                                        self.cfg.head_dim, np.arange(n)))
+    def _rope_rows(self, pos) -> tuple:
+        """cos and sin of the positions' angles, on the GPU."""
+        return tuple(torch.from_numpy(a).to(self.dev) for a in
+                     rope_cos_sin(self.cfg.rope_theta, self.cfg.head_dim,
+                                  pos))
 
     def _send(self, arrays) -> List[torch.Tensor]:
         """The arrays as int32 device tensors, in one copy (each starts on
@@ -172,13 +174,14 @@ class HipBackend:
             chain.from_iterable(chain.from_iterable(
                 it.write_positions for it in items)),
             np.uint32).reshape(-1, 2)
+        rope = None
         if rows and int(pos.max()) >= self._rope[0].shape[0]:
-            self._rope_rows(1 << int(pos.max()).bit_length())
+            rope = self._rope_rows(pos)  # (past the table: these rows alone)
         toks, pos, sb, so, tables, offs, reads, last = self._send(
             [toks, pos, slots[:, 0], slots[:, 1], padded_tables(items),
              first, np.array([it.read_num_tokens for it in items], np.int64),
              last])
-        cos, sin = (t.index_select(0, pos) for t in self._rope)
+        cos, sin = rope or (t.index_select(0, pos) for t in self._rope)
         x = w["embed"][toks]
         scale = 1.0 / math.sqrt(hd)
         decode = not last_only and bool((n_new == 1).all())

@@ -2424,6 +2424,25 @@ def test_backend_rope_table_grows():
     assert torch.equal(*out)
 
 
+def test_backend_forward_computes_no_other_rope_rows(monkeypatch):
+    """A forward computes no angles at the positions that the context holds,
+    and past it those of its own rows alone."""
+    from rvllm_amd import attn_model
+    from rvllm_amd.engine import BatchItem
+    cfg = attn_model.AttnModelConfig(context_length=8192)
+    be = attn_model.HipBackend(cfg, attn_model.init_weights(cfg), 20, 1024)
+    asked, rope = [], attn_model.rope_cos_sin
+    monkeypatch.setattr(
+        attn_model, "rope_cos_sin",
+        lambda theta, hd, pos: asked.append(len(pos)) or rope(theta, hd, pos))
+    for p in (4095, 4096, 8191, 8192, 9000):
+        items = [BatchItem(0, [5], [(p // 1024, p % 1024)], list(range(10)),
+                           p + 1, p),
+                 BatchItem(1, [9], [(12, 1)], [12], 2, 1)]
+        be.forward_sample(items, False, [None] * 2)
+    assert asked == [2, 2]  # (the last two steps)
+
+
 @pytest.mark.parametrize("rows,V", [(1, 4096), (1, 16388), (511, 4100),
                                     (512, 4100), (700, 1003), (2, 4101)])
 def test_argmax_thread_counts(rows, V):

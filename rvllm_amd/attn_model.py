@@ -209,8 +209,11 @@ class HipBackend:
                 r0 = 0
                 for i, it in enumerate(items):  # one prefill item at a time
                     n = len(it.tokens)
+                    # (its own blocks: by the batch's width a short prompt
+                    # would be taken for a chunk behind a long context)
+                    w_i = max(1, len(it.read_blocks))
                     st.paged_prefill(l, qr[r0:r0 + n].view(1, n, H, hd),
-                                     tables[i:i + 1], offs[i:i + 1],
+                                     tables[i:i + 1, :w_i], offs[i:i + 1],
                                      reads[i:i + 1],
                                      out=att[r0:r0 + n].view(1, n, H, hd),
                                      scale=scale, window=c.window)

@@ -2443,6 +2443,38 @@ def test_backend_forward_computes_no_other_rope_rows(monkeypatch):
     assert asked == [2, 2]  # (the last two steps)
 
 
+def test_backend_prompts_by_their_own_tables(monkeypatch):
+    """A prompt of a batch is computed as it is alone, whatever longer ones
+    stand beside it: the same table width (which decides whether its keys are
+    cut into pieces) and the same attention bits."""
+    from rvllm_amd.attn_model import AttnModelConfig, HipBackend, init_weights
+    from rvllm_amd.engine import BatchItem
+    cfg = AttnModelConfig(n_layers=1, n_heads=32, n_kv_heads=8)
+    be = HipBackend(cfg, init_weights(cfg), 200, 16)
+    seen, prefill = [], be.st.paged_prefill
+
+    def record(layer, q, tables, *args, **kw):
+        out = prefill(layer, q, tables, *args, **kw)
+        seen.append((tables.shape[1], q.clone(), out.clone()))
+        return out
+
+    monkeypatch.setattr(be.st, "paged_prefill", record)
+    rng = np.random.default_rng(0)
+    items, at = [], 0
+    for i, n in enumerate((900, 754, 411)):
+        blocks = list(range(at, at + -(-n // 16)))
+        at += len(blocks)
+        items.append(BatchItem(i, rng.integers(0, cfg.vocab, n).tolist(),
+                               [(blocks[p // 16], p % 16) for p in range(n)],
+                               blocks, n, 0))
+    be.forward_sample(items, True, [None] * 3)
+    assert [w for w, _, _ in seen] == [len(it.read_blocks) for it in items]
+    for (w, q, out), it in zip(list(seen), items):
+        alone = prefill(0, q, dev_u32([it.read_blocks]), dev_u32([0]),
+                        dev_u32([len(it.tokens)]))
+        assert torch.equal(out, alone)
+
+
 @pytest.mark.parametrize("rows,V", [(1, 4096), (1, 16388), (511, 4100),
                                     (512, 4100), (700, 1003), (2, 4101)])
 def test_argmax_thread_counts(rows, V):

@@ -1831,24 +1831,29 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
   uint32_t n_sub, gt;
   subgroups(group ? group : 1, &n_sub, &gt);
   const uint64_t pairs = (uint64_t)batch * p->n_kv * n_sub;
-  // Two workgroups a CU, in whole 64-token steps (2 x 12345 tokens of
-  // Qwen3-0.6B heads: 448 partitions' workgroups 20.9 us, the next power of
-  // two's 400 21.4 us; 8 x 5000, f32 cells: 512 against 320, 53.3 against
-  // 57.8 us; for 768 or 1024 workgroups the same or slower). At least 256
-  // tokens, or 128 where a key is 1 KiB (3 x 600 tokens of gemma-3 heads:
-  // 17.2 -> 11.1 us). Large groups at head_dim 256 keep powers of two and no
-  // other rule: rvkv_paged_decode_noalloc refuses them by their partials'
-  // size, which stays what it is.
+  // Two workgroups a CU, at least 256 tokens each (128 where a key is 1 KiB:
+  // 3 x 600 tokens of gemma-3 heads 17.2 -> 11.1 us), in powers of two, or
+  // finer in whole 64-token steps where that makes no more than 512 workgroups
+  // (2 x 12345 tokens of Qwen3-0.6B heads: 448 20.9 us, the power of two's 400
+  // 21.4; 14 x 12000 128 -> 114, log-uniformly spread 72 -> 57; 150 log-uniform
+  // gemma-3 sequences to 1100, f32, 47.6 -> 40.0). A few past 512 run in a
+  // second round, or at half the waves (launch_decode): 14 x 4000 Qwen3 tokens
+  // 560 49.1 us, 448 44.1; 120 x 4000 of gemma-3 600 114.5, 480 91.4. Large
+  // groups at head_dim 256 keep powers of two and no other rule:
+  // rvkv_paged_decode_noalloc refuses them by their partials' size, which stays
+  // what it is.
   const uint64_t want = 512;
-  const uint64_t parts = pairs >= want ? 1 : (want + pairs - 1) / pairs;
-  const uint64_t per = (max_ctx + parts - 1) / parts;
   const bool big = p->head_dim > 128;
-  uint64_t P = big && gt <= 4 ? 128 : 256;
-  if (big && gt > 4) {
-    while (P < per && P < (1u << 30)) P <<= 1;
-    return (uint32_t)P;
+  const uint64_t least = big && gt <= 4 ? 128 : 256;
+  uint64_t parts = pairs >= want ? 1 : (want + pairs - 1) / pairs;
+  uint64_t P = least;
+  while (P < (max_ctx + parts - 1) / parts && P < (1u << 30)) P <<= 1;
+  if (big && gt > 4) return (uint32_t)P;
+  if (parts > 1) {
+    parts = std::max<uint64_t>(want / pairs, 2);
+    const uint64_t fine = ((max_ctx + parts - 1) / parts + 63) / 64 * 64;
+    P = std::max(least, std::min(P, fine));
   }
-  P = std::max<uint64_t>(P, (per + 63) / 64 * 64);
   // (a ragged batch holds perhaps 40 % of what its longest sequence says)
   if (one_workgroup(p, decode_rate(p, n_heads, gt), max_ctx, P,
                     0.4 * max_ctx * pairs))

@@ -1778,6 +1778,22 @@ def test_decode_partition_rule(hd, G, batch, ctx, dtype):
 
 
 @pytest.mark.parametrize("hd,nkv,G,dtype", [
+    (128, 8, 2, torch.float16), (256, 1, 4, torch.float16),
+    (256, 1, 4, torch.float32), (64, 5, 3, torch.float32)])
+def test_decode_partitions_of_one_generation(hd, nkv, G, dtype):
+    """Partitions make at most 512 workgroups (two a CU) where a sequence gets
+    more than two, or are a power of two that long: a few workgroups past that
+    run in a second round."""
+    st = HipKvStorage(1, 1, 16, nkv, hd, dtype=dtype)
+    for batch in (1, 3, 14, 20, 31, 60, 100, 120, 170, 255):
+        for ctx in (700, 2000, 4000, 12345, 100000):
+            P = st.decode_partition_tokens(batch, nkv * G, ctx)
+            parts = -(-ctx // P)
+            assert (parts <= 2 or parts * batch * nkv <= 512 or
+                    P & (P - 1) == 0), (batch, ctx, P)
+
+
+@pytest.mark.parametrize("hd,nkv,G,dtype", [
     (128, 8, 2, torch.float16), (256, 1, 4, torch.float32),
     (256, 2, 8, torch.float16), (64, 5, 3, torch.float32)])
 def test_decode_unbounded_max_ctx_len(hd, nkv, G, dtype):

@@ -1761,12 +1761,14 @@ uint32_t env_u32(const char *name) {
   return v ? (uint32_t)strtoul(v, nullptr, 10) : 0u;
 }
 
-// KB/us that one decode workgroup streams where the chip is idle: eight and
-// more waves, four, or four on the matrix cores (a wave's 32-key tiles follow
-// each other).
-double decode_rate(const rvkv_pool *p, uint32_t n_heads, uint32_t gt) {
+// KB/us that one of `wgs` decode workgroups streams where the chip is idle:
+// eight and more waves (launch_decode gives them to at most 256 workgroups),
+// four, or four on the matrix cores (a wave's 32-key tiles follow each other).
+double decode_rate(const rvkv_pool *p, uint32_t n_heads, uint32_t gt,
+                   uint64_t wgs) {
   if (rvkv_detail::mfma_decode_wanted(p, n_heads)) return 29e3;
-  return decode_max_waves((int)decode_hd(p->head_dim), (int)gt, p->f32()) > 4
+  return wgs <= 256 && decode_max_waves((int)decode_hd(p->head_dim), (int)gt,
+                                        p->f32()) > 4
              ? 60e3
              : 40e3;
 }
@@ -1776,16 +1778,40 @@ double decode_rate(const rvkv_pool *p, uint32_t n_heads, uint32_t gt) {
 // than in partitions of `part` tokens: cutting costs the reduction launch,
 // ~5 us; the chip streams 5.3 MB/us. (us a layer, cut with the reduction and
 // its launch gap against one: SmolLM2 heads f32, 8 x 512, 14.3 / 9.6;
-// Qwen3-0.6B heads 1 x 500 13.9 / 10.3, 1 x 1000 12.3 / 14.7, 20 x 1500
-// 31.0 / 25.9, 40 x 4500 170 / 141; gemma-3 heads f32, 100 ragged to 1500,
-// 42 / 59. Matrix cores, Llama-3.2-1B heads: 4 x 400 11.3 / 8.6, 4 x 760 13.1
-// / 11.8, 40 x 630 25.5 / 16.5, 1 x 1000 12.3 / 13.)
+// Qwen3-0.6B heads 1 x 500 13.9 / 10.3, 1 x 1000 12.3 / 14.7. Matrix cores,
+// Llama-3.2-1B heads: 4 x 400 11.3 / 8.6, 4 x 760 13.1 / 11.8, 40 x 630
+// 25.5 / 16.5, 1 x 1000 12.3 / 13.)
 bool one_workgroup(const rvkv_pool *p, double rate, double longest,
                    double part, double all) {
   const double row = 2.0 * p->head_dim * p->elem_bytes;  // bytes a token
   const double shared = row * all / 5.3e6;
   return std::max(row * longest / rate, shared) <=
          std::max(row * std::min(part, longest) / rate, shared) + 5.0;
+}
+
+// The VALU decode without a plan, where two partitions a sequence would do
+// (171-511 workgroups): whether one partition is no slower, whatever the
+// batch's lengths are. Measured at 26-60 sequences of Qwen3-0.6B, 44-90 of
+// SmolLM2 (f32) and 240-480 of gemma-3 (f16, f32) heads, to 700, 2000, 4000
+// and 12000 tokens, all alike, evenly and log-uniformly spread:
+//  - f16 rows of 512 bytes: 0-40 % faster at any length; past 256 workgroups
+//    two partitions run two waves each (launch_decode), one runs four (gemma-3
+//    log-uniform, 240 x 4000 129.8 -> 124.2 us, 400 x 2000 130.0 -> 109.1).
+//  - Up to 256 workgroups, which get eight waves: to 2048 tokens 0-16 %
+//    faster; to 4000, 28 log-uniform Qwen3 sequences 42.2 -> 46.4.
+//  - From 416 workgroups (four waves; two partitions leave a third of the
+//    chip's second generation idle): to 4096 tokens 7 % faster to 2 % slower;
+//    60 log-uniform sequences to 8000 122 -> 128.
+//  - Between, the CUs that hold two workgroups set the time: 40 Qwen3
+//    sequences to 2000 61.4 -> 64.0 alike, 31.9 -> 37.6 log-uniform; to 8000
+//    98.6 -> 121.6.
+bool one_of_two(const rvkv_pool *p, uint32_t gt, uint64_t pairs,
+                uint32_t max_ctx) {
+  const bool wide = decode_max_waves((int)decode_hd(p->head_dim), (int)gt,
+                                     p->f32()) > 4;
+  if (!p->f32() && p->head_dim > 128 && gt <= 4) return true;
+  if (pairs <= 256) return wide && max_ctx <= 2048;
+  return pairs >= 416 && max_ctx <= 4096;
 }
 
 // The matrix-core decode without a plan: waves a partition (its keys split
@@ -1812,7 +1838,7 @@ uint32_t mfma_uniform_parts(const rvkv_pool *p, uint32_t n_heads,
   uint32_t P = 256;
   while (P < per && P < 4096) P <<= 1;
   if (*ksplit == 4 && max_ctx <= 4096 &&
-      one_workgroup(p, decode_rate(p, n_heads, 1), max_ctx, P,
+      one_workgroup(p, decode_rate(p, n_heads, 1, pairs), max_ctx, P,
                     0.4 * max_ctx * pairs))
     P = std::max(P, (max_ctx + 255) / 256 * 256);
   return P;
@@ -1854,9 +1880,9 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
     const uint64_t fine = ((max_ctx + parts - 1) / parts + 63) / 64 * 64;
     P = std::max(least, std::min(P, fine));
   }
-  // (a ragged batch holds perhaps 40 % of what its longest sequence says)
-  if (one_workgroup(p, decode_rate(p, n_heads, gt), max_ctx, P,
-                    0.4 * max_ctx * pairs))
+  // (Nothing is known of the other sequences: they may all be short.)
+  if (one_workgroup(p, decode_rate(p, n_heads, gt, pairs), max_ctx, P, 0) ||
+      (parts == 2 && one_of_two(p, gt, pairs, max_ctx)))
     P = std::max<uint64_t>(P, ((uint64_t)max_ctx + 63) / 64 * 64);
   // (a bound near 2^32, "none", must not round up to 0 in 32 bits)
   return (uint32_t)std::min<uint64_t>(P, 1u << 30);
@@ -2520,7 +2546,7 @@ int plan_build(rvkv_decode_plan *pl, const uint32_t *ctx_lens_host,
   // reduction would cost more (Qwen3-0.6B heads, 30 ragged to 1500: 24.3 ->
   // 22.1 us; Llama-3.2-1B heads, 8 ragged to 500: 14 -> 9.4 us).
   if (batch * n_hy <= 512 &&
-      one_workgroup(pool, decode_rate(pool, pl->n_heads, gt), longest, P,
+      one_workgroup(pool, decode_rate(pool, pl->n_heads, gt, 1), longest, P,
                     (double)total * n_hy))
     whole_max = longest;
   auto split = [&](uint32_t start, uint32_t n, uint32_t *step_out) {

@@ -1793,6 +1793,20 @@ def test_decode_partitions_of_one_generation(hd, nkv, G, dtype):
                     P & (P - 1) == 0), (batch, ctx, P)
 
 
+@pytest.mark.parametrize("hd,nkv,G,dtype,most", [
+    (128, 8, 2, torch.float16, 51), (64, 5, 3, torch.float32, 83),
+    (256, 1, 4, torch.float16, 170), (256, 1, 4, torch.float32, 415)])
+def test_decode_long_sequence_alone_is_cut(hd, nkv, G, dtype, most):
+    """A batch may hold one long sequence among short ones: it is cut in every
+    batch where partitions shorten the launch (a workgroup streams 40-60 KB a
+    us, the reduction takes 5 us)."""
+    st = HipKvStorage(1, 1, 16, nkv, hd, dtype=dtype)
+    for batch in range(1, most + 1):
+        for ctx in (5000, 8000, 16000):
+            P = st.decode_partition_tokens(batch, nkv * G, ctx)
+            assert P <= (ctx + 1) // 2 + 63, (batch, ctx, P)
+
+
 @pytest.mark.parametrize("hd,nkv,G,dtype", [
     (128, 8, 2, torch.float16), (256, 1, 4, torch.float32),
     (256, 2, 8, torch.float16), (64, 5, 3, torch.float32)])

@@ -2544,10 +2544,15 @@ int plan_build(rvkv_decode_plan *pl, const uint32_t *ctx_lens_host,
                                 2.0 * P);
   // A launch that leaves workgroup slots idle: no sequence is cut where the
   // reduction would cost more (Qwen3-0.6B heads, 30 ragged to 1500: 24.3 ->
-  // 22.1 us; Llama-3.2-1B heads, 8 ragged to 500: 14 -> 9.4 us).
-  if (batch * n_hy <= 512 &&
-      one_workgroup(pool, decode_rate(pool, pl->n_heads, gt, 1), longest, P,
-                    (double)total * n_hy))
+  // 22.1 us; Llama-3.2-1B heads, 8 ragged to 500: 14 -> 9.4 us). VALU decode:
+  // up to 256 workgroups, which get eight waves (300 log-uniform gemma-3
+  // sequences to 300 18.8 us cut, 21.7 whole), and by the longest sequence's
+  // own time against the longest item's, as the others do not hide it (by the
+  // whole batch's bytes: 50 log-uniform Qwen3 sequences to 8000 74.8 -> 141 us,
+  // 20 evenly spread to 8000 80.7 -> 90.9).
+  if (batch * n_hy <= (mfma ? 512u : 256u) &&
+      one_workgroup(pool, decode_rate(pool, pl->n_heads, gt, 1), longest,
+                    std::max(P, whole_max), mfma ? (double)total * n_hy : 0))
     whole_max = longest;
   auto split = [&](uint32_t start, uint32_t n, uint32_t *step_out) {
     const uint32_t span = n - start;

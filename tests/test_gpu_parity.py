@@ -1807,6 +1807,18 @@ def test_decode_long_sequence_alone_is_cut(hd, nkv, G, dtype, most):
             assert P <= (ctx + 1) // 2 + 63, (batch, ctx, P)
 
 
+@pytest.mark.parametrize("batch", [20, 36, 50, 62])
+def test_plan_long_sequence_alone_is_cut(batch):
+    """A plan cuts a long sequence among short ones, which set the launch's
+    time alone otherwise, and keeps short ones whole."""
+    st = HipKvStorage(1, 1, 16, 8, 128)
+    short = np.linspace(30, 500, batch).astype(int)
+    assert HipDecodePlan(st, short, 16).items == batch
+    for top in (2000, 8000):
+        lens = np.exp(np.linspace(np.log(30), np.log(top), batch)).astype(int)
+        assert HipDecodePlan(st, lens, 16).items > batch, top
+
+
 @pytest.mark.parametrize("hd,nkv,G,dtype", [
     (128, 8, 2, torch.float16), (256, 1, 4, torch.float32),
     (256, 2, 8, torch.float16), (64, 5, 3, torch.float32)])

@@ -1298,7 +1298,14 @@ __global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, false))
 // A lane loads 4 cells (16 bytes) per row and load, NL loads per row: R =
 // HD / (4 NL) lanes per row, RPL = 64 / R rows per wave-wide load. Masked
 // keys load zero rows, as in the f16 kernel.
-template <int HD, int GT>
+//
+// AHEAD: the appended row is loaded ahead of the loop, for launches that leave
+// the chip idle (a short context's whole time is a few round trips to memory:
+// 30 x 512 tokens of SmolLM2 heads 11.7 -> 11.1 us, 8 x 512 10.55 -> 10.4).
+// Where the chip is full, its registers cost a resident wave (gemma-3 heads,
+// 300 log-uniform sequences to 4000 264 -> 292 us), and so they do at head_dim
+// 256 everywhere (8 x 512 the same either way).
+template <int HD, int GT, bool AHEAD>
 __global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, true))
     decode_f32_kernel(const uint4 *p_items, const uint32_t *p_tables,
                       const uint32_t *p_ctx, uint32_t p_mb, uint32_t p_bs,
@@ -1399,14 +1406,14 @@ __global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, true))
   const uint32_t newtok = (a.new_k != nullptr && ctx - 1 >= t0 && ctx - 1 < t1)
                               ? ctx - 1
                               : 0xFFFFFFFFu;
-  // The appended row and its slot are loaded ahead of the loop: a short
-  // context's whole time is a few round trips to memory.
   const bool has_new = newtok != 0xFFFFFFFFu && wave == 0;
   float4 nk[NL], nv[NL];
   uint32_t new_blk = 0, new_off = 0;
   if (has_new) {
     new_blk = sload(a.new_blk + b);
     new_off = sload(a.new_off + b);
+  }
+  auto load_new = [&]() {
     const size_t src = ((size_t)b * a.n_kv + kvh) * HD;
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
@@ -1429,7 +1436,8 @@ __global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, true))
                             (float)v23.y);
       }
     }
-  }
+  };
+  if (AHEAD && has_new) load_new();
   // Block ids by scalar loads, a chunk ahead.
   auto fetch_ids = [&](uint32_t ch) {
 #pragma unroll
@@ -1502,6 +1510,7 @@ __global__ void __launch_bounds__(64 * decode_max_waves(HD, GT, true))
     }
   }
   if (has_new) {
+    if constexpr (!AHEAD) load_new();
     // The appended row (f32 source copied, f16 widened exactly, as the
     // append does): stored by sub-group 0's row group 0, and one more key
     // of row group 0's softmax state.
@@ -1985,10 +1994,14 @@ void launch_decode(const DecodeArgs &a, dim3 grid, hipStream_t st) {
   // least the f32 kernel's W * GT * (HD + 2) floats.
   const size_t lds =
       (((size_t)W * GT * 2 + 3) / 4 * 4 + (size_t)W * GT * HD) * sizeof(float);
-  if (a.f32cache)
-    hipLaunchKernelGGL((decode_f32_kernel<HD, GT>), grid, dim3(64 * W), lds, st,
-                       a.items, a.tables, a.ctx_lens, a.max_blocks, a.bs_log2,
-                       a.part_tokens, a);
+  if (a.f32cache && HD <= 128 && wgs <= 256)
+    hipLaunchKernelGGL((decode_f32_kernel<HD, GT, HD <= 128>), grid,
+                       dim3(64 * W), lds, st, a.items, a.tables, a.ctx_lens,
+                       a.max_blocks, a.bs_log2, a.part_tokens, a);
+  else if (a.f32cache)
+    hipLaunchKernelGGL((decode_f32_kernel<HD, GT, false>), grid, dim3(64 * W),
+                       lds, st, a.items, a.tables, a.ctx_lens, a.max_blocks,
+                       a.bs_log2, a.part_tokens, a);
   else if (a.hd != HD)  // a head_dim below HD: rows read element by element
     hipLaunchKernelGGL((decode_part_kernel<HD, GT, 4, 1, true>), grid,
                        dim3(64 * W), lds, st, a.items, a.tables,

@@ -404,3 +404,34 @@ def test_f32_prefill_position_near_2_32():
         for off in (2 ** 32 - 1, 2 ** 32 - 5, 2 ** 31):
             out = st.paged_prefill(0, q, t, dev_u32([off]), dev_u32([n]))
             assert torch.equal(out, want), off
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128, 256])
+@pytest.mark.parametrize("batch", [128, 129])  # 256 workgroups, and more
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+def test_f32_decode_step_appended_row(hd, batch, dtype):
+    """The appended row loaded ahead of the keys and after them: the f32
+    decode of the step and the row in the cache, against float64 (f32 products
+    and sums: 2e-5)."""
+    nkv, bs, mb = 2, 16, 6
+    st = HipKvStorage(1, batch * mb, bs, nkv, hd, dtype=torch.float32)
+    at = np.arange(batch * mb * bs)
+    rnd = lambda *s: torch.randn(*s, device="cuda")
+    st.write_tokens(0, dev_u32(at // bs), dev_u32(at % bs),
+                    rnd(len(at), nkv, hd), rnd(len(at), nkv, hd))
+    rng = np.random.default_rng(hd)
+    tables = rng.permutation(batch * mb).reshape(batch, mb).astype(np.uint32)
+    lens = rng.integers(1, mb * bs + 1, batch)
+    lens[:3] = 1, 64, mb * bs
+    pos = lens - 1
+    k, v = (rnd(batch, nkv, hd).to(dtype) for _ in range(2))
+    q = rnd(batch, nkv * 3, hd)
+    blk = tables[np.arange(batch), pos // bs]
+    out = st.decode_step(0, k, v, dev_u32(blk), dev_u32(pos % bs), q,
+                         dev_u32(tables), dev_u32(lens), mb * bs)
+    for w, x in ((0, k), (1, v)):
+        got = st.read_blocks(0, w, dev_u32(blk))
+        assert torch.equal(got[range(batch), pos % bs], x.float())
+    from tests.test_gpu_parity import _prefill_f64
+    want = _prefill_f64(st, q[:, None], tables, pos, lens, 0)
+    assert (out - want[:, 0]).abs().max() < 2e-5

@@ -435,3 +435,77 @@ def test_f32_decode_step_appended_row(hd, batch, dtype):
     from tests.test_gpu_parity import _prefill_f64
     want = _prefill_f64(st, q[:, None], tables, pos, lens, 0)
     assert (out - want[:, 0]).abs().max() < 2e-5
+
+
+@pytest.mark.parametrize("hd", [64, 256])
+def test_f32_prefill_cut_keys_streams_and_capture(hd):
+    """Calls queued on three streams at once (the first two cut the keys, the
+    third does not) and a captured one (not cut) replayed between them: each
+    against float64 (f32 products and sums: 2e-5)."""
+    Q, nkv, H, bs, prior = 40, 1, 4, 16, 3000
+    n = prior + Q
+    nb = -(-n // bs)
+    table = np.random.default_rng(hd).permutation(nb).astype(np.uint32)
+    at = np.arange(n)
+    st = HipKvStorage(1, nb, bs, nkv, hd, dtype=torch.float32)
+    st.write_tokens(0, dev_u32(table[at // bs]), dev_u32(at % bs),
+                    *(torch.randn(n, nkv, hd, device="cuda")
+                      for _ in range(2)))
+    t, p, r = dev_u32(table[None]), dev_u32([prior]), dev_u32([n])
+    qs = [torch.randn(1, Q, H, hd, device="cuda") for _ in range(4)]
+    want = [_prefill_f64_of(st, q, table, prior, n) for q in qs]
+    outs = [torch.empty_like(q) for q in qs]
+    own, streams = st.stream, [torch.cuda.Stream() for _ in range(3)]
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        st.set_stream(torch.cuda.current_stream())
+        st.paged_prefill(0, qs[3], t, p, r, out=outs[3])
+    for _ in range(3):
+        for o in outs:
+            o.zero_()
+        torch.cuda.synchronize()
+        for q, o, s in zip(qs, outs, streams):
+            st.set_stream(s)
+            st.paged_prefill(0, q, t, p, r, out=o)
+        graph.replay()
+        torch.cuda.synchronize()
+        for o, w in zip(outs, want):
+            assert (o - w).abs().max() < 2e-5
+    st.set_stream(own)
+    assert torch.equal(*(st.paged_prefill(0, qs[0], t, p, r)
+                         for _ in range(2)))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_whole_sequence_plan_with_appended_row(dtype):
+    """A plan that keeps sequences whole past its item size (30 ragged ones to
+    1500), with the step's rows appended: against float64, and the rows in the
+    cache."""
+    from rvllm_amd.kv_storage import HipDecodePlan
+    from tests.test_gpu_parity import _prefill_f64
+    nkv, G, hd, bs, batch, mb = 8, 2, 128, 16, 30, 94
+    st = HipKvStorage(1, batch * mb, bs, nkv, hd, dtype=dtype)
+    at = np.arange(batch * mb * bs)
+    rnd = lambda *s: torch.randn(*s, device="cuda").to(dtype)
+    st.write_tokens(0, dev_u32(at // bs), dev_u32(at % bs),
+                    rnd(len(at), nkv, hd), rnd(len(at), nkv, hd))
+    rng = np.random.default_rng(5)
+    tables = rng.permutation(batch * mb).reshape(batch, mb).astype(np.uint32)
+    lens = np.linspace(100, 1500, batch).astype(int)
+    pos = lens - 1
+    plan = HipDecodePlan(st, lens, nkv * G)
+    if dtype == torch.float16:  # (an f32 row is twice the bytes)
+        assert plan.items == batch
+    k, v = (torch.randn(batch, nkv, hd, device="cuda") for _ in range(2))
+    q = torch.randn(batch, nkv * G, hd, device="cuda")
+    blk = tables[np.arange(batch), pos // bs]
+    out = st.decode_step(0, k, v, dev_u32(blk), dev_u32(pos % bs), q,
+                         dev_u32(tables), dev_u32(lens), plan=plan)
+    for w, x in ((0, k), (1, v)):
+        got = st.read_blocks(0, w, dev_u32(blk))[range(batch), pos % bs]
+        assert torch.equal(got, x.to(dtype))
+    want = _prefill_f64(st, q[:, None], tables, pos, lens, 0)
+    # (f16: probabilities and packed products in f16, as every decode test)
+    tol = 2e-5 if dtype == torch.float32 else 2e-3
+    assert (out - want[:, 0]).abs().max() < tol

@@ -77,7 +77,8 @@ int rvkv_pool_create(uint32_t n_layers, uint32_t num_blocks,
                      uint32_t head_dim, rvkv_dtype cache_dtype,
                      rvkv_stream stream, rvkv_pool **out);
 void rvkv_pool_destroy(rvkv_pool *pool);
-/* Bytes of device memory the pool holds (K+V, all layers). */
+/* Bytes of the pool's cache (K+V, all layers), without the scratch behind
+ * it. */
 size_t rvkv_pool_bytes(const rvkv_pool *pool);
 /* Rebinds the pool to another stream on the same device. */
 int rvkv_pool_set_stream(rvkv_pool *pool, rvkv_stream stream);
@@ -312,9 +313,13 @@ int rvkv_attn_prep(rvkv_pool *pool, uint32_t layer, const float *q_in,
  * arithmetic. Allocates nothing. Calls whose query rows alone leave the GPU
  * idle are cut along the keys and merged by a second launch; the partial
  * results go to the pool's scratch, half of which the first two streams that
- * such calls run on get each. On further streams, on hipStreamPerThread and
- * under graph capture the keys are not cut (the same result to within
- * rounding). */
+ * such calls run on get each, for the pool's life: also once they are
+ * destroyed (a stream is idle before it is destroyed, as a later one may get
+ * its handle). On further streams, on hipStreamPerThread and under graph
+ * capture the keys are not cut (the same result to within rounding). The
+ * pieces are sized by max_blocks, the bound that the host knows: a table far
+ * wider than the context pays for the second launch without need (~3 us), so
+ * pass it no wider than the longest sequence's blocks. */
 int rvkv_paged_prefill(rvkv_pool *pool, uint32_t layer, const float *q,
                        const uint32_t *block_tables,
                        const uint32_t *pos_offset,

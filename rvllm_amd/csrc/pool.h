@@ -27,8 +27,9 @@ struct rvkv_pool {
   // Scratch for the partial results of prefills that are cut along their
   // keys: kSplitStreams regions of kSplitBytes behind the cache tensors, in
   // the same allocation (NULL if there was no room for them). A region
-  // belongs to the first stream that used it, for the pool's life, so two
-  // streams never share one and calls need no ordering between streams.
+  // belongs to the first stream that used it, for the pool's life (a stream
+  // may be destroyed long before the pool learns of it), so two streams never
+  // share one and calls need no ordering between streams.
   unsigned char *split_base;
   hipStream_t split_stream[2];
   uint32_t n_split;

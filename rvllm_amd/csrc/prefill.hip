@@ -1244,13 +1244,18 @@ __global__ void __launch_bounds__(
 // cycles for a 16 KiB tile (head_dim 64), so staging it in LDS for several
 // waves would save loads that nothing waits for. The next tile's K loads go
 // out behind the S product and its V loads behind P.V, into the registers
-// just read. Bound by the matrix cores (53 % busy; the rest is each wave's
-// ~6 us of start-up and merge and the last, partly filled generation).
-// Against one wave a (query head, row) in plain FMAs: SmolLM2 heads, one
-// prompt of 700 rows 777 -> 31 us a layer; Llama-3.2-1B heads, 1500 rows
-// 118 us (78 TFLOP/s). One, two or four waves a row tile: 700 rows 61, 44,
-// 31 us, 1500 rows 187, 125, 118 us. At three waves a SIMD (168 registers)
-// it spills: 155 us; two S chains instead of one: 119 us.
+// just read. Bound by each wave's chain of dependent tiles (load, S, softmax,
+// P.V) at one or two waves a SIMD: 700 rows of SmolLM2 heads keep the matrix
+// cores 21 % busy, the waves wait 44 % of their cycles, and 330 workgroups load
+// 256 CUs unevenly; 1500 rows of Llama-3.2-1B heads reach 78 TFLOP/s, half of
+// what a large f32 product reaches. Against one wave a (query head, row) in
+// plain FMAs: SmolLM2 heads, one prompt of 700 rows 777 -> 31 us a layer;
+// Llama-3.2-1B heads, 1500 rows 117 us. One, two or four waves a row tile: 700
+// rows 61, 44, 31 us, 1500 rows 187, 125, 117 us. At three waves a SIMD (168
+// registers) it spills: 155 us; two S chains instead of one: 119 us. The block
+// ids (three sets of eight) fill the scalar registers: 27-34 spill at head_dim
+// 64, 104-111 at 128 and 260-278 at 256, where 20-27 vector registers do too
+// (76-88 bytes of scratch a lane).
 constexpr int kF32Rows = 32, kF32Keys = 32, kF32Waves = 4;
 // At head_dim 256 the registers hold O and one of K and V: Q is in LDS, and
 // each tile's K and V are loaded when they are needed.

@@ -3,9 +3,10 @@
 rope_cos_sin follows src/model.rs:224-250: theta_j = rope_theta **
 (-2 j / head_dim), divided by factors[j] when Llama-3 frequency factors are
 given; angle[i, j] = positions[i] * theta_j; the tables are cos and sin of
-the angles, f32 [n, head_dim / 2]. Like the reference, the table is built
-once per forward on the host (positions are host-side bookkeeping) and
-shared by every layer; it is a few KB per step, not part of the hot path.
+the angles, f32 [n, head_dim / 2], computed on the host. The reference builds
+it once per forward for that forward's positions; the engine backend builds it
+once for all positions of the context and gathers a forward's rows on the GPU.
+Every layer shares them.
 """
 from __future__ import annotations
 

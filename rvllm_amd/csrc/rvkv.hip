@@ -1855,6 +1855,7 @@ uint32_t mfma_uniform_parts(const rvkv_pool *p, uint32_t n_heads,
 
 uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
                           uint32_t max_ctx) {
+  batch = std::max(batch, 1u);  // (an empty batch: any size)
   static const uint32_t forced = env_u32("RVKV_DECODE_PART_TOKENS");
   if (forced >= 256 && forced % 256 == 0) return forced;
   if (rvkv_detail::mfma_decode_wanted(p, n_heads)) {

@@ -509,3 +509,18 @@ def test_whole_sequence_plan_with_appended_row(dtype):
     # (f16: probabilities and packed products in f16, as every decode test)
     tol = 2e-5 if dtype == torch.float32 else 2e-3
     assert (out - want[:, 0]).abs().max() < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("hd,G", [(128, 2), (64, 4), (256, 8)])
+def test_decode_empty_batch(hd, G, dtype):
+    """The size queries answer for an empty batch (no partials), and a decode
+    of one returns at once."""
+    st = HipKvStorage(1, 4, 16, 1, hd, dtype=dtype)
+    for ctx in (0, 1, 5000):
+        assert st.decode_partition_tokens(0, G, ctx) > 0
+        assert st.decode_workspace_bytes(0, G, ctx) == 0
+    none = torch.empty(0, dtype=torch.int32, device="cuda")
+    out = st.paged_decode(0, torch.empty(0, G, hd, device="cuda"),
+                          none.view(0, 4), none, 5000)
+    assert out.shape == (0, G, hd)

@@ -1873,9 +1873,9 @@ uint32_t partition_tokens(const rvkv_pool *p, uint32_t batch, uint32_t n_heads,
   // (2 x 12345 tokens of Qwen3-0.6B heads: 448 20.9 us, the power of two's 400
   // 21.4; 14 x 12000 128 -> 114, log-uniformly spread 72 -> 57; 150 log-uniform
   // gemma-3 sequences to 1100, f32, 47.6 -> 40.0). A few past 512 run in a
-  // second round, or at half the waves (launch_decode): 14 x 4000 Qwen3 tokens
-  // 560 49.1 us, 448 44.1; 120 x 4000 of gemma-3 600 114.5, 480 91.4. Large
-  // groups at head_dim 256 keep powers of two and no other rule:
+  // second generation, or at half the waves (launch_decode): 14 x 4000 Qwen3
+  // tokens 560 49.1 us, 448 44.1; 120 x 4000 of gemma-3 600 114.5, 480 91.4.
+  // Large groups at head_dim 256 keep powers of two and no other rule:
   // rvkv_paged_decode_noalloc refuses them by their partials' size, which stays
   // what it is.
   const uint64_t want = 512;

@@ -1783,7 +1783,7 @@ def test_decode_partition_rule(hd, G, batch, ctx, dtype):
 def test_decode_partitions_of_one_generation(hd, nkv, G, dtype):
     """Partitions make at most 512 workgroups (two a CU) where a sequence gets
     more than two, or are a power of two that long: a few workgroups past that
-    run in a second round."""
+    run in a second generation."""
     st = HipKvStorage(1, 1, 16, nkv, hd, dtype=dtype)
     for batch in (1, 3, 14, 20, 31, 60, 100, 120, 170, 255):
         for ctx in (700, 2000, 4000, 12345, 100000):
